@@ -30,7 +30,7 @@ EXPORTS = [
     "fl_state_force_timeout",
     "fl_decode_step", "fl_decode_sample", "fl_decode_hidden", "fl_verify", "fl_kv_move", "fl_sample",
     "fl_sample_noalloc", "fl_probe_handoff", "fl_tile_int4", "fl_dequant_int4_tiled", "fl_gemv_int4_tiled",
-    "fl_probe_dequant",
+    "fl_probe_dequant", "fl_gemm_rows_workspace", "fl_gemm_rows_int4",
 ]
 
 
@@ -83,6 +83,8 @@ def load(path=LIB_PATH):
         "fl_dequant_int4_mx": ([vp, vp, vp, i32, i32, vp], i32),
         "fl_gemv_int4": ([vp, vp, vp, vp, i32, i32, vp], i32),
         "fl_gemm_int4": ([vp, vp, vp, vp, i32, i32, i32, vp], i32),
+        "fl_gemm_rows_workspace": ([i32, i32, i32, ctypes.POINTER(ctypes.c_int64)], i32),
+        "fl_gemm_rows_int4": ([vp, vp, vp, vp, vp, i32, i32, i32, vp], i32),
         "fl_state_create": ([ctypes.POINTER(ModelDesc), i32, vp, vp, ctypes.POINTER(vp)], i32),
         "fl_state_destroy": ([vp], i32),
         "fl_state_reset": ([vp, vp], i32),

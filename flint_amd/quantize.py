@@ -80,8 +80,9 @@ def gemv_int4(q, sz, x, y=None):
 
 
 def gemm_int4(q, sz, x, y=None):
-    """Y[M,N] = bf16(X[M,K] . dq[N,K]^T) for any M: blocks of up to 32 rows (FL_MAX_VERIFY), each
-    one fl_gemm_int4 launch that reads the weights once for all of its rows."""
+    """Y[M,N] = bf16(X[M,K] . dq[N,K]^T) for any M: one fl_gemm_int4 launch up to 32 rows
+    (FL_MAX_VERIFY), which reads the weights once for all of them; beyond, fl_gemm_rows_int4, which
+    reads and dequantises them once per 64 or 128 rows."""
     _check_dev(q, torch.int32, "q")
     _check_dev(sz, torch.int32, "sz")
     _check_dev(x, torch.bfloat16, "x")
@@ -93,6 +94,13 @@ def gemm_int4(q, sz, x, y=None):
         y = torch.empty(m, n, dtype=torch.bfloat16, device=q.device)
     if m > 0 and (y.shape != (m, n) or not y.is_contiguous()):
         raise ValueError("y must be a contiguous [M, N] tensor")
+    if m > _lib.MAX_VERIFY:
+        need = _lib.ctypes.c_int64()
+        if _lib.load().fl_gemm_rows_workspace(m, n, k, _lib.ctypes.byref(need)) == _lib.FL_OK:
+            ws = torch.empty(need.value // 4, dtype=torch.float32, device=q.device) if need.value else None
+            _lib.call("fl_gemm_rows_int4", _lib.ptr(q), _lib.ptr(sz), _lib.ptr(x), _lib.ptr(y), _lib.ptr(ws),
+                      m, n, k, _lib.stream_ptr())
+            return y
     for r0 in range(0, m, _lib.MAX_VERIFY):
         mb = min(_lib.MAX_VERIFY, m - r0)
         _lib.call("fl_gemm_int4", _lib.ptr(q), _lib.ptr(sz), _lib.ptr(x[r0:]), _lib.ptr(y[r0:]), mb, n, k,
@@ -137,8 +145,8 @@ def scales_and_zeros_gptfast(sz):
 class WeightOnlyInt4Linear(torch.nn.Module):
     """Drop-in for reference engine/quantize.py:483-525 (groupsize 128), on the HIP GEMVs.
 
-    forward(x [..., K] bf16) -> [..., N] bf16; M = prod(leading dims) <= 32 rows per call
-    (one weight read for all rows), as in decode and speculative verify; more rows raise.
+    forward(x [..., K] bf16) -> [..., N] bf16 for any M = prod(leading dims): the GEMV at M = 1, one
+    weight read for up to 32 rows (speculative verify), the tiled GEMM for more (a prompt).
     """
 
     def __init__(self, in_features, out_features, bias=False, device=None, groupsize=GROUP):

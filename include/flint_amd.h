@@ -103,6 +103,16 @@ int fl_gemv_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint1
 int fl_gemm_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint16_t* y,
                  int32_t m, int32_t n, int32_t k, void* stream);
 
+/* The same product for any M >= 1 (a whole prompt through one layer): tiles of 64 or 128 rows of
+ * both operands on the matrix cores, each weight dequantised once per 64 or 128 rows of X. ws: device
+ * workspace of at least the bytes that fl_gemm_rows_workspace gives for (m, n, k) (0: may be NULL),
+ * 16-byte aligned, free for reuse once the call's work on the stream is done. FL_E_ARG for a size
+ * that they do not take (K > 65536, or N K / 2 beyond 4 GB).
+ * Replaces reference engine/quantize.py:517-525 WeightOnlyInt4Linear.forward on a prompt. */
+int fl_gemm_rows_workspace(int32_t m, int32_t n, int32_t k, int64_t* bytes);
+int fl_gemm_rows_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint16_t* y, float* ws,
+                      int32_t m, int32_t n, int32_t k, void* stream);
+
 /* ---- tiled layout: the exact dequantisation on the matrix cores ------------------------- */
 
 /* The same int4 values in the tiled layout the matrix-core kernels read (N % 16 == 0): per block

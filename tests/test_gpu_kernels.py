@@ -190,6 +190,29 @@ def test_weight_only_int4_linear(dev, lead):
         mod(torch.zeros(4, k + 128, dtype=torch.bfloat16, device=dev))  # wrong inner dimension
 
 
+@pytest.mark.parametrize("m,n,k", [(33, 64, 128), (64, 63, 384), (65, 2570, 2560), (127, 130, 8192), (129, 16385, 256),
+                                   (300, 16384, 128), (2049, 2048, 384), (8193, 65, 128)])
+def test_gemm_rows(dev, m, n, k):
+    """fl_gemm_rows_int4 at the edges of its tiles (64 and 128 rows of both operands), of its K
+    parts and of its launches of 8192 rows, N odd and not, into an output that is not 8-byte aligned
+    too: fp32 sums of exact products, so a result may differ from the oracle's only where another
+    order of the sum rounds to the neighbouring bf16 value."""
+    from flint_amd.quantize import dequantize_int4, gemm_int4, quantize_int4
+    w = _weights(n, k, 21, "edge").to(dev)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(22)).to(torch.bfloat16).to(dev)
+    q, sz = quantize_int4(w)
+    ref = x.float() @ dequantize_int4(q, sz).float().T
+    # |fp32 sum - exact| <= K 2^-24 sum |x w|, and half a bf16 ulp of the result
+    bound = k * 2.0 ** -23 * (x.float().abs() @ dequantize_int4(q, sz).float().abs().T) + ref.abs() * 2.0 ** -8
+    y = gemm_int4(q, sz, x)
+    d = (y.float() - ref).abs()
+    log(f"gemm rows {m} x {n} x {k}: max|d| {float(d.max()):.3e}, largest share of its bound {float((d / bound).max()):.3f}")
+    assert bool((d <= bound).all())
+    buf = torch.zeros(m * n + 3, dtype=torch.bfloat16, device=dev)
+    gemm_int4(q, sz, x, buf[1:1 + m * n].view(m, n))
+    assert torch.equal(buf[1:1 + m * n].view(m, n), y) and not buf[:1].any() and not buf[1 + m * n:].any()
+
+
 def test_scales_and_zeros_gptfast_layout(dev):
     """scales_and_zeros_gptfast gives gpt-fast's [K/128, N, 2] bf16 tensor
     (reference engine/quantize.py:79-93 pack_scales_and_zeros) of the same values the oracle

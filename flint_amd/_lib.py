@@ -31,6 +31,7 @@ EXPORTS = [
     "fl_decode_step", "fl_decode_sample", "fl_decode_hidden", "fl_verify", "fl_kv_move", "fl_sample",
     "fl_sample_noalloc", "fl_probe_handoff", "fl_tile_int4", "fl_dequant_int4_tiled", "fl_gemv_int4_tiled",
     "fl_probe_dequant", "fl_gemm_rows_workspace", "fl_gemm_rows_int4",
+    "fl_prefill_workspace", "fl_prefill",
 ]
 
 
@@ -98,6 +99,8 @@ def load(path=LIB_PATH):
         "fl_decode_sample": ([ctypes.POINTER(Weights), vp, vp, i32, f32, i32, ctypes.c_uint64, ctypes.c_uint64,
                               vp, vp, vp, vp], i32),
         "fl_verify": ([ctypes.POINTER(Weights), vp, vp, i32, vp, vp, i32, vp, vp, vp, vp], i32),
+        "fl_prefill_workspace": ([vp, i32, ctypes.POINTER(ctypes.c_int64)], i32),
+        "fl_prefill": ([ctypes.POINTER(Weights), vp, vp, i32, i32, vp, vp, vp], i32),
         "fl_kv_move": ([vp, vp, vp, i32, vp], i32),
         "fl_sample": ([vp, i32, i32, f32, i32, ctypes.c_uint64, ctypes.c_uint64, vp, vp, vp, vp], i32),
         "fl_sample_noalloc": ([vp, i32, i32, f32, i32, ctypes.c_uint64, ctypes.c_uint64, vp, vp, vp, vp], i32),

@@ -11,7 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libflint_amd.so")
 OBJDIR = os.path.join(HERE, "_build")
-SOURCES = ["fl_quant.hip", "fl_decode.hip", "fl_sample.hip", "fl_probe.hip", "fl_tiled.hip", "fl_gemm.hip"]
+SOURCES = ["fl_quant.hip", "fl_decode.hip", "fl_sample.hip", "fl_probe.hip", "fl_tiled.hip", "fl_gemm.hip", "fl_prefill.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
@@ -25,7 +25,7 @@ FLAGS = [
 
 # per-source extra flags: the MFMA-dequant kernels keep their matrix-core results in VGPRs (the
 # accumulation registers would cost a copy per result read by the vector ALUs)
-EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("fl_tiled.hip", "fl_gemm.hip")}
+EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("fl_tiled.hip", "fl_gemm.hip", "fl_prefill.hip")}
 
 
 def _compile(src):

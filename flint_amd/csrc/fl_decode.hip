@@ -28,7 +28,7 @@
 //    slices (long contexts only) publish tagged partials that slice 0 merges in order.
 // The speculative-verify kernel (k_verify, below) runs M tokens through the same protocol with
 // the GEMMs on the matrix cores.
-#include "fl_common.h"
+#include "fl_state.h"
 #include <stdlib.h>
 #include <string.h>
 #include <mutex>
@@ -3367,50 +3367,6 @@ int phase_fits(int n, int k, int G, int cap, int mode) {
 
 }  // namespace
 
-struct fl_state {
-  fl_model_desc d;
-  int max_seq;
-  int grid;   // decode workgroups (1 per CU)
-  int vgrid;  // verify workgroups (1 per CU)
-  uint16_t *kc, *vc;
-  uint32_t *h, *attn, *act;
-  unsigned long long* qkv;
-  unsigned long long* part;
-  uint16_t* vrows;              // verify exchange rows: h [FL_MAX_VERIFY][D], attn [..][D], act [..][F]
-  unsigned long long* vpart;    // verify attention slice partials [NH][VNS][FL_MAX_VERIFY][66]
-  uint32_t* vflag;              // verify ready flags
-  uint32_t* shist;              // fused sampling exchange: per-workgroup histograms
-  unsigned long long* sword;    // ... bin totals, maxima, partial sums
-  int att_spw, gq_min, gq_kps;
-  int defer_min;  // key slices from which the per-head attention leaves its merge to the O phase
-  int vkps, vtok_work;
-  int coop;       // launch with hipLaunchCooperativeKernel (else a plain launch, the default)
-  // the k_decode instantiations of the chunk budget that fits the model, by attention: per-head
-  // units (0), with the slice merge deferred to the O phase (1), by KV group (2; small budget only,
-  // else null)
-  const void* kdec[3];
-  int verify_ok;  // k_verify's dynamic LDS fits and a grid of it is co-resident
-  unsigned long long* amax;
-  uint32_t* done;
-  int32_t* err;
-  uint32_t epoch;
-  unsigned long long* prof;
-  int prof_slots;
-  unsigned long long spin_ticks;  // wait bound passed to every launch
-  uint32_t* stall;                // zero word, never written: forced-timeout wait (tests)
-  int force_timeout;
-  void* blocks[16];
-  int nblocks;
-  void* uc[12];  // pooled uncached exchange buffers
-  size_t uc_bytes[12];
-  int nuc;
-  // Tags are 16 bits (1..65535) and advance 5 per layer per launch, so a word left over from an
-  // older launch could carry the tag a reader is waiting for once the tags have gone round. The
-  // exchange buffers are zeroed (tag 0: never valid) every clear_period launches, fewer than
-  // take the tags round.
-  uint32_t clear_period, since_clear;
-};
-
 namespace {
 __global__ __launch_bounds__(256) void k_zero(uint4* __restrict__ p, size_t n16) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256)
@@ -3500,13 +3456,13 @@ void uc_release(void* v) {
 }
 }  // namespace
 
-namespace {
-bool weights_ok(const fl_weights* w) {
+bool fl_weights_ok(const fl_weights* w) {
   return w && w->wqkv_q && w->wqkv_sz && w->wo_q && w->wo_sz && w->wgu_q && w->wgu_sz && w->wd_q &&
          w->wd_sz && w->attn_norm && w->ffn_norm && w->final_norm && w->embed && w->rope &&
          w->rope_len > 0;
 }
 
+namespace {
 DecodeParams base_params(const fl_weights* w, fl_state* st, int pos) {
   DecodeParams p;
   memset(&p, 0, sizeof(p));
@@ -3826,20 +3782,20 @@ int fl_kv_move(fl_state* st, const int32_t* src, const int32_t* dst, int32_t n, 
 
 int fl_decode_step(const fl_weights* w, fl_state* st, const int32_t* token_in, int32_t pos,
                    int32_t* token_out, float* logits, uint16_t* feat, void* stream) {
-  if (!st || !token_in || !token_out || !weights_ok(w)) return FL_E_ARG;
+  if (!st || !token_in || !token_out || !fl_weights_ok(w)) return FL_E_ARG;
   return decode_launch(w, st, token_in, nullptr, pos, token_out, logits, feat, stream);
 }
 
 int fl_decode_hidden(const fl_weights* w, fl_state* st, uint16_t* h, int32_t pos,
                      int32_t* token_out, float* logits, uint16_t* feat, void* stream) {
-  if (!st || !h || !weights_ok(w)) return FL_E_ARG;
+  if (!st || !h || !fl_weights_ok(w)) return FL_E_ARG;
   return decode_launch(w, st, nullptr, h, pos, token_out, logits, feat, stream);
 }
 
 int fl_decode_sample(const fl_weights* w, fl_state* st, const int32_t* token_in, int32_t pos,
                      float temperature, int32_t top_k, uint64_t seed, uint64_t offset,
                      int32_t* token_out, float* logits, uint16_t* feat, void* stream) {
-  if (!st || !token_in || !token_out || !weights_ok(w) || top_k < 0) return FL_E_ARG;
+  if (!st || !token_in || !token_out || !fl_weights_ok(w) || top_k < 0) return FL_E_ARG;
   if (!(temperature == temperature) || st->d.vocab > 65536) return FL_E_ARG;
   // one LM-head row per thread of a workgroup in the sampling epilogue
   {
@@ -3855,7 +3811,7 @@ int fl_decode_sample(const fl_weights* w, fl_state* st, const int32_t* token_in,
 int fl_verify(const fl_weights* w, fl_state* st, const int32_t* tokens, int32_t m,
               const int32_t* depth, const uint8_t* amask, int32_t pos, int32_t* tokens_out,
               float* logits, uint16_t* feat, void* stream) {
-  if (!st || !tokens || !depth || !amask || !tokens_out || !weights_ok(w)) return FL_E_ARG;
+  if (!st || !tokens || !depth || !amask || !tokens_out || !fl_weights_ok(w)) return FL_E_ARG;
   if (!w->wqkv_t || !w->wo_t || !w->wgu_t || !w->wd_t) return FL_E_ARG;  // verify reads the tiled copies
   if (m < 1 || m > FL_MAX_VERIFY) return FL_E_M;
   if (pos < 0 || pos + m > st->max_seq) return FL_E_POS;

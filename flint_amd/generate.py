@@ -8,13 +8,18 @@ is prefilled through the speculative-verify kernel, up to 32 tokens per launch.
 """
 import torch
 
+# prompts of more tokens than this run as fl_prefill passes (flint-3b, 40 layers: 32 tokens 3.28 ms in a
+# pass and 3.19 in a verify launch, 40 tokens 3.30 and 4.82)
+PREFILL_MIN = 32
+
 
 def prefill(model, x, input_pos, chunk=32):
     """Feed prompt tokens x (int32 device [T]) at positions input_pos[0]..; returns the greedy next
     token (int32 device [1]) after the last one (reference engine/generate.py:57-60, which runs
-    the prompt through one forward). The prompt goes through the verify kernel `chunk` (<= 32)
-    tokens per launch with a causal mask: each launch reads every weight once for the whole
-    chunk and appends the chunk's K/V rows."""
+    the prompt through one forward). With the default chunk, more than PREFILL_MIN tokens go through
+    fl_prefill, up to 1024 per pass. Fewer, or a smaller chunk, go through the verify kernel
+    `chunk` (<= 32) tokens per launch with a causal mask: each launch reads every weight once for
+    the whole chunk and appends the chunk's K/V rows."""
     from . import _lib
     x = x.reshape(-1).to(device=model.device, dtype=torch.int32)
     p0 = int(input_pos.reshape(-1)[0]) if torch.is_tensor(input_pos) else int(input_pos)
@@ -23,6 +28,11 @@ def prefill(model, x, input_pos, chunk=32):
     out = torch.empty(1, dtype=torch.int32, device=model.device)
     if n == 0:
         return out
+    if chunk == _lib.MAX_VERIFY and n > PREFILL_MIN and hasattr(model, "prefill"):
+        try:
+            return model.prefill(x, p0, out)
+        except torch.OutOfMemoryError:
+            pass  # no room for its workspace: the verify launches need none
     cache = getattr(model, "_prefill_masks", None)
     if cache is None:
         cache = model._prefill_masks = {}

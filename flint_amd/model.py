@@ -281,6 +281,23 @@ class Transformer:
                   _lib.ptr(tokens_out), _lib.ptr(logits), _lib.ptr(feat), _lib.stream_ptr())
         return tokens_out, logits, feat
 
+    def prefill(self, tokens, pos, token_out):
+        """A prompt (int32 device [n]) at cache slots pos..pos+n-1 in passes of up to 1024 tokens
+        (fl_prefill): fills the cache and writes the greedy next token to token_out (int32 device
+        [1]), which it returns. The workspace (84 MB for 1024 tokens of flint-3b) is torch's."""
+        if self._state is None:
+            raise RuntimeError("call setup_caches first")
+        tokens = tokens.contiguous()
+        for t, nm in ((tokens, "tokens"), (token_out, "token_out")):
+            if not t.is_cuda or t.dtype != torch.int32:
+                raise ValueError(f"{nm} must be a {torch.int32} device tensor")
+        n, need = tokens.numel(), _lib.ctypes.c_int64()
+        _lib.call("fl_prefill_workspace", self._state, n, _lib.ctypes.byref(need))
+        ws = torch.empty(need.value, dtype=torch.uint8, device=self.device)
+        _lib.call("fl_prefill", _lib.ctypes.byref(self._cw), self._state, _lib.ptr(tokens), n, int(pos),
+                  _lib.ptr(token_out), _lib.ptr(ws), _lib.stream_ptr())
+        return token_out
+
     def kv_move(self, src, dst):
         """Move the K/V rows of cache slots src[i] to dst[i] in every layer (host int lists, at most
         32): the KV compaction after a tree verify (reference spec_tree.py:124-127). All rows are

@@ -217,6 +217,19 @@ int fl_verify(const fl_weights* w, fl_state* st, const int32_t* tokens, int32_t 
               const int32_t* depth, const uint8_t* amask, int32_t pos,
               int32_t* tokens_out, float* logits, uint16_t* feat, void* stream);
 
+/* A prompt of n >= 1 tokens at cache slots pos..pos+n-1 with a causal mask: K/V rows of every layer
+ * into the cache, the greedy next token after the last one to *token_out. The same operations as
+ * fl_verify, in ordinary launches over up to 1024 tokens at a time; it takes the models that
+ * fl_verify takes and needs the tiled weight copies. workspace: device memory of the bytes that
+ * fl_prefill_workspace gives for n (84 MB for 1024 tokens of flint-3b), 256-byte aligned, free for
+ * reuse once the call's work on the stream is done. tokens / token_out are device pointers; a
+ * token id outside the vocabulary is recorded in the state (fl_state_check). Nothing is allocated, and
+ * a captured call replays (no tags).
+ * Replaces reference engine/generate.py:57-60 prefill (one forward over the prompt). */
+int fl_prefill_workspace(fl_state* st, int32_t n, int64_t* bytes);
+int fl_prefill(const fl_weights* w, fl_state* st, const int32_t* tokens, int32_t n, int32_t pos,
+               int32_t* token_out, void* workspace, void* stream);
+
 /* KV cache compaction after a tree verify: for i = 0..n-1 (n <= FL_MAX_VERIFY) the K and V rows
  * of cache slot src[i] move to slot dst[i], in every layer and KV group. All n rows are read
  * before any is written, which equals moving them one at a time in order i whenever no source is

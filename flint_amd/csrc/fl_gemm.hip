@@ -1,4 +1,5 @@
-// int4 linear over more rows than one fl_gemm_int4 launch takes (a prompt through one layer).
+// The int4 linear for more than one row: fl_gemm_int4 (up to 32 rows: speculative verify) and
+// fl_gemm_rows_int4 (any number: a prompt through one layer).
 #include "fl_gemm.h"
 #include <algorithm>
 
@@ -32,37 +33,64 @@ struct EpiPart {
 };
 
 // y = bf16(the partial sums, added in order); one thread per four columns
-__global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ p, uint16_t* __restrict__ y, int m,
-                                                   int n, int np, int splits, bool vec) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, total = (size_t)m * (np >> 2);
+__global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ p, EpiBf16 out, int np, int splits) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, total = (size_t)out.m * (np >> 2);
   if (i >= total) return;
   const int mm = (int)(i / (np >> 2)), nn = 4 * (int)(i % (np >> 2));
   fl_f32x4 v = *reinterpret_cast<const fl_f32x4*>(p + (size_t)mm * np + nn);
-  for (int s = 1; s < splits; ++s) v += *reinterpret_cast<const fl_f32x4*>(p + ((size_t)s * m + mm) * np + nn);
-  EpiBf16{y, m, n, vec}(nn, mm, v, 0);
+  for (int s = 1; s < splits; ++s) v += *reinterpret_cast<const fl_f32x4*>(p + ((size_t)s * out.m + mm) * np + nn);
+  out(nn, mm, v, 0);
 }
 
 // How a call of m rows runs. 128 x 128 tiles where they fill the chip (256 CUs, two workgroups each):
-// 512 / 2048 rows x 16384 x 2560 took 60 / 235 us, 64 x 64 tiles 75 / 290. Else 64 x 64 tiles, K cut
-// until there are about 768 workgroups of at least four 128-groups: 64 x 2560 x 8192 took 49 us
-// uncut, 16 us in 4 parts and 13 in 8; 336 x 2576 x 2560 (246 tiles) 24 uncut, 17 in 2 and 15 in 4;
-// 512 x 3584 x 2560 (448 tiles) 25 uncut and 23 in 2, less than the second launch that adds the
-// parts costs (3-4 us).
+// 512 / 2048 rows x 16384 x 2560 took 60 / 235 us, 64 x 64 tiles 75 / 290. Else 64 x 64 tiles:
+// - up to 64 rows: four ways, and K cut until there are about 192 workgroups of at least four
+//   128-groups: 64 x 16384 x 2560 took 18 us with one way and 15 with four, 64 x 2560 x 8192 (40 tiles)
+//   36 us uncut and 12 in four parts;
+// - K cut until there are about 768 workgroups: 336 x 2576 x 2560 (246 tiles) took 24 us uncut, 17 in
+//   2 parts and 15 in 4; but from 320 tiles and for few groups two ways instead, as the launch that
+//   adds the parts costs 3-4 us: 512 x 2560 x 2560 (320 tiles) took 25 us with one way uncut, 20 in
+//   2 parts and 20 with two ways uncut, 512 x 3584 x 2560 (448 tiles) 25, 23 and 21.
 struct Plan {
   bool big;
-  int splits, gps;
+  int ways, splits, gps;
 };
 Plan plan_rows(int m, int n, int k) {
   const int G = k / FL_GROUP;
-  Plan p{true, 1, G};
+  Plan p{true, 1, 1, G};
   if ((int64_t)((m + 127) / 128) * ((n + 127) / 128) >= 256) return p;
   p.big = false;
   const int64_t tiles = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
-  int s = (int)std::min<int64_t>(8, std::max<int64_t>(1, 768 / tiles));
-  s = std::max(1, std::min(s, G / 4));
-  p.gps = (G + s - 1) / s;
+  int64_t s = 768 / tiles, most = 8;
+  if (m <= 64) {
+    p.ways = 4;
+    s = 192 / tiles;
+    most = 4;
+  } else if (tiles >= 320 && G <= 32) {
+    p.ways = 2;
+    s = 1;
+  }
+  const int parts = (int)std::max<int64_t>(1, std::min({most, s, (int64_t)G / 4}));
+  p.gps = (G + parts - 1) / parts;
   p.splits = (G + p.gps - 1) / p.gps;
   return p;
+}
+
+template <int NW, int KW, int NB, int MB, class Epi>
+void launch(GemmArgs a, Epi epi, hipStream_t s) {
+  a.nblk = (a.n + 16 * NW * NB - 1) / (16 * NW * NB);
+  a.mblk = (a.m + 16 * MB - 1) / (16 * MB);
+  hipLaunchKernelGGL((k_gemm_rows<false, NW, KW, NB, MB, 1, 1, Epi>), dim3(gemm_grid(a)), dim3(64 * NW * KW), 0, s, a, epi);
+}
+template <class Epi>
+void launch_small(int ways, const GemmArgs& a, Epi epi, hipStream_t s) {
+  if (ways == 4) launch<4, 4, 1, 4>(a, epi, s);
+  else if (ways == 2) launch<4, 2, 1, 4>(a, epi, s);
+  else launch<4, 1, 1, 4>(a, epi, s);
+}
+
+EpiBf16 out_bf16(uint16_t* y, int m, int n) {
+  return EpiBf16{y, m, n, n % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0};
 }
 
 // rows of one launch: 32-bit byte offsets over X (and the rows of a last tile past its end)
@@ -74,6 +102,29 @@ bool rows_ok(int n, int k) {
 }  // namespace
 
 extern "C" {
+
+int fl_gemm_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint16_t* y, int32_t m, int32_t n,
+                 int32_t k, void* stream) {
+  if (!q || !sz || !x || !y || n <= 0 || k <= 0 || (k % FL_GROUP) != 0) return FL_E_ARG;
+  if (m < 1 || m > FL_MAX_VERIFY) return FL_E_M;
+  if ((int64_t)n * (k / 2) > 0xFFFFFFFFll || (int64_t)m * k * 2 > 0xFFFFFFFFll) return FL_E_ARG;
+  const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const GemmArgs a{q, sz, x, m, n, k, 0, 0, 1, k / FL_GROUP};
+  const EpiBf16 epi = out_bf16(y, m, n);
+  // One workgroup per 64 weight rows (four ways) where that gives at least 192, else one per 16 rows
+  // with as many ways as the LDS holds: 32 rows x 16384 x 2560 12 us (four ways; 23 in the former
+  // kernel, which re-read X from L2 per 16 weight rows), 5 rows x 2560 x 8192 9.7 us (sixteen ways;
+  // 12.2, four waves whose 16 loads each waited for the one before), 32 rows 13.7 us (eight ways).
+  const bool wide = (n + 63) / 64 >= 192;
+  if (m <= 16) {
+    if (wide) launch<4, 4, 1, 1>(a, epi, s);
+    else launch<1, 16, 1, 1>(a, epi, s);
+  } else {
+    if (wide) launch<4, 4, 1, 2>(a, epi, s);
+    else launch<1, 8, 1, 2>(a, epi, s);
+  }
+  return hipGetLastError() == hipSuccess ? FL_OK : FL_E_LAUNCH;
+}
 
 int fl_gemm_rows_workspace(int32_t m, int32_t n, int32_t k, int64_t* bytes) {
   if (!bytes || m < 1 || n < 1 || k < 1 || k % FL_GROUP || !rows_ok(n, k)) return FL_E_ARG;
@@ -97,22 +148,16 @@ int fl_gemm_rows_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, 
   for (int r0 = 0; r0 < m; r0 += ROWS_PER_LAUNCH) {
     const int rows = std::min(ROWS_PER_LAUNCH, m - r0);
     const Plan p = plan_rows(rows, n, k);
-    const int t = p.big ? 128 : 64;
-    uint16_t* yr = y + (size_t)r0 * n;
-    const bool vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(yr) & 7) == 0;
-    GemmArgs a{q, sz, x + (size_t)r0 * k, rows, n, k, (n + t - 1) / t, (rows + t - 1) / t, p.splits, p.gps};
+    const EpiBf16 epi = out_bf16(y + (size_t)r0 * n, rows, n);
+    const GemmArgs a{q, sz, x + (size_t)r0 * k, rows, n, k, 0, 0, p.splits, p.gps};
     if (p.big) {
-      hipLaunchKernelGGL((k_gemm_rows<false, 4, 2, 8, EpiBf16>), dim3(gemm_grid(a)), dim3(256), 0, s, a,
-                         EpiBf16{yr, rows, n, vec});
+      launch<4, 1, 2, 8>(a, epi, s);
     } else if (p.splits == 1) {
-      hipLaunchKernelGGL((k_gemm_rows<false, 4, 1, 4, EpiBf16>), dim3(gemm_grid(a)), dim3(256), 0, s, a,
-                         EpiBf16{yr, rows, n, vec});
+      launch_small(p.ways, a, epi, s);
     } else {
-      hipLaunchKernelGGL((k_gemm_rows<false, 4, 1, 4, EpiPart>), dim3(gemm_grid(a)), dim3(256), 0, s, a,
-                         EpiPart{ws, rows, np});
+      launch_small(p.ways, a, EpiPart{ws, rows, np}, s);
       const size_t quads = (size_t)rows * (np / 4);
-      hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, ws, yr, rows, n, np,
-                         p.splits, vec);
+      hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s, ws, epi, np, p.splits);
     }
   }
   return hipGetLastError() == hipSuccess ? FL_OK : FL_E_LAUNCH;

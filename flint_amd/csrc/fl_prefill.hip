@@ -6,10 +6,10 @@
 //   residual + RMSNorm -> gate/up GEMM (SwiGLU in its epilogue) -> down GEMM -> residual + RMSNorm,
 // the O and down GEMMs cut along K into fp32 part sums that the residual kernel adds in order. After
 // the last pass the LM head and argmax of the last token.
-// At 512 tokens of flint-3b a layer takes 174 us (of which the GEMMs: QKV 28, O 20, gate/up 60, down 47;
-// attention 17, the two norms 15), against 1336 in sixteen k_verify launches; 33 tokens take 82 us a
-// layer (launches and latency) against 120, and up to 32 the one k_verify launch is faster (n = 32:
-// 80 us a layer against 82, at 4000 cached keys 98 against 113).
+// At 512 tokens of flint-3b a layer takes 170 us (of which the GEMMs: QKV 24, O 20, gate/up 57, down 44;
+// attention 17, the two norms 13), against 1336 in sixteen k_verify launches; 40 tokens take 64 us a
+// layer (launches and latency) against 120, and up to 32 they take the one k_verify launch (n = 16:
+// 46 us a layer against 61; n = 32: 80 against 62, but at 12000 cached keys 125 against 150).
 #include "fl_gemm.h"
 #include "fl_state.h"
 #include <algorithm>
@@ -412,35 +412,43 @@ PfWs pf_layout(const fl_model_desc& d, int T, uint8_t* base) {
   return w;
 }
 
-// K parts of a GEMM whose part sums are added by k_pf_norm: enough workgroups for about two per CU of
-// at least four 128-groups each
-int pf_splits(int tiles, int groups) {
-  return std::max(1, std::min({PF_SPLITS, 512 / std::max(1, tiles), groups / 4}));
+template <int NW, int KW, int MB, class Epi>
+void pf_launch(GemmArgs a, Epi epi, hipStream_t s) {
+  a.nblk = (a.n + 16 * NW - 1) / (16 * NW);
+  a.mblk = (a.m + 16 * MB - 1) / (16 * MB);
+  constexpr int D = KW == 1 ? 2 : 1;  // groups requested ahead
+  hipLaunchKernelGGL((k_gemm_rows<true, NW, KW, 1, MB, D, D, Epi>), dim3(gemm_grid(a)), dim3(64 * NW * KW), 0, s, a, epi);
 }
 
-// 128 x 128 tiles (eight waves) where they give at least 160 workgroups, or with parts to add, from
-// 128 tokens; 64 x 64 tiles else
+// One GEMM of a pass, in 64 x 64 tiles (four waves a way) or 128 x 128 (eight). `parts`: the epilogue
+// keeps fp32 sums of K parts, which k_pf_norm adds; returns their number. Measured at flint-3b's
+// sizes (us):
+// - up to 256 tiles of 64 four ways, up to 512 two: QKV at 64 / 512 tokens (56 / 448 tiles) 19 / 28 with one
+//   way, 12 / - with four, - / 21 with two; gate/up at 64 (256) 20 and 13, at 100 (512) 24 and 21;
+// - more: tiles of 128 if those are at least 160 (gate/up at 512 tokens 58, 64 x 64 tiles 75), else 64;
+// - parts of 64 x 64 tiles: about ten groups each, four at most, more while they give fewer than 160
+//   workgroups. O at 512 tokens (320 tiles) 18 us in two parts, 17 in four, whose sums cost more to add;
+//   down 41 in four, 47 in two; at 64 tokens O 7 in four, down 11 in four with four ways, 16 with one;
+// - parts of 128 x 128 tiles: two workgroups per CU. At 1024 tokens (160 tiles; 640 of 64) O 27 us in
+//   three parts and 31 in two, down 65 in three and 71 in four.
 template <class Epi>
 int pf_gemm(const uint32_t* qt, const uint32_t* sz, const uint16_t* x, int T, int n, int k, bool parts, Epi epi,
             hipStream_t s) {
   const int G = k / FL_GROUP;
   GemmArgs a{qt, sz, x, T, n, k, 0, 0, 1, G};
-  auto tiles = [&](int t) {
-    a.nblk = (n + t - 1) / t;
-    a.mblk = (T + t - 1) / t;
-    return a.nblk * a.mblk;
-  };
-  const bool big = T > 64 && (tiles(128) >= 160 || parts);
-  const int nt = tiles(big ? 128 : 64);
+  const int t64 = ((n + 63) / 64) * ((T + 63) / 64), t128 = ((n + 127) / 128) * ((T + 127) / 128);
+  const bool big = t64 > 512 && t128 >= 160;
   if (parts) {
-    a.splits = pf_splits(nt, G);
+    const int want = big ? 512 / t128 : std::max(G / 10, (160 + t64 - 1) / t64);
+    a.splits = std::max(1, std::min({PF_SPLITS, want, G / 4}));
     a.gps = (G + a.splits - 1) / a.splits;
     a.splits = (G + a.gps - 1) / a.gps;
   }
-  if (big)
-    hipLaunchKernelGGL((k_gemm_rows<true, 8, 1, 8, Epi>), dim3(gemm_grid(a)), dim3(512), 0, s, a, epi);
-  else
-    hipLaunchKernelGGL((k_gemm_rows<true, 4, 1, 4, Epi>), dim3(gemm_grid(a)), dim3(256), 0, s, a, epi);
+  const int wgs = t64 * a.splits;
+  if (big) pf_launch<8, 1, 8>(a, epi, s);
+  else if (wgs <= 256 && a.gps >= 8) pf_launch<4, 4, 4>(a, epi, s);
+  else if (wgs <= 512 && a.gps >= 8) pf_launch<4, 2, 4>(a, epi, s);
+  else pf_launch<4, 1, 4>(a, epi, s);
   return a.splits;
 }
 

@@ -8,8 +8,8 @@ is prefilled through the speculative-verify kernel, up to 32 tokens per launch.
 """
 import torch
 
-# prompts of more tokens than this run as fl_prefill passes (flint-3b, 40 layers: 32 tokens 3.28 ms in a
-# pass and 3.19 in a verify launch, 40 tokens 3.30 and 4.82)
+# prompts of more tokens than this run as fl_prefill passes (flint-3b, 40 layers: 40 tokens 2.55 ms in a
+# pass and 4.81 in two verify launches; 32 tokens in one launch 3.2 ms, at 12000 cached keys 5.0 against 6.1)
 PREFILL_MIN = 32
 
 

@@ -31,33 +31,37 @@
 
 namespace {
 
-// row layout -> tiled layout: one thread per 16-byte tiled chunk
+// row layout -> tiled layout: a workgroup takes four units (16 rows x one 128-group each), stages their
+// words in LDS with coalesced 16-byte loads, and each thread gathers one 16-byte tiled chunk from
+// there. 16384 x 2560 took 21.6 us (1.9 TB/s) with the gathers going to global memory, 32 loads per
+// thread that each used one nibble; now 9 us (4.7 TB/s).
+constexpr int TL_LD = 68;  // words per staged row: rows 4p + j start 16 p + 4 j banks apart
 __global__ __launch_bounds__(256) void k_tile_int4(const uint32_t* __restrict__ q, uint4* __restrict__ qt,
                                                    int n, int k) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int G = k >> 7;
-  const int64_t chunks = (int64_t)(n >> 4) * G * 64;
-  if (idx >= chunks) return;
-  const int l = (int)(idx & 63), p = (l >> 2) & 3, c = 4 * (l >> 4) + (l & 3);
-  const int64_t blk = idx >> 6;
-  const int g = (int)(blk % G), rb = (int)(blk / G);
-  const int kw = k >> 3;  // words per row
-  auto nib = [&](int r, int col) -> uint32_t {  // q[r][col] of the row layout
-    const uint32_t w = q[(size_t)r * kw + (col >> 3)];
-    return (w >> (4 * nib_pos(col & 7))) & 0xFu;
-  };
+  __shared__ __align__(16) uint32_t ws[16 * TL_LD];
+  const int G = k >> 7, gb = (G + 3) >> 2, tid = threadIdx.x;
+  const int rb = (int)(blockIdx.x / gb), g0 = 4 * (int)(blockIdx.x % gb);
+  {
+    const int row = tid >> 4, ch = tid & 15;
+    if (g0 + (ch >> 2) < G)
+      *reinterpret_cast<uint4*>(ws + row * TL_LD + 4 * ch) =
+          *reinterpret_cast<const uint4*>(q + ((size_t)rb * 16 + row) * (k >> 3) + (size_t)g0 * 16 + 4 * ch);
+  }
+  __syncthreads();
+  const int u = tid >> 6, l = tid & 63, p = (l >> 2) & 3, c = 4 * (l >> 4) + (l & 3);
+  if (g0 + u >= G) return;
+  const uint32_t* src = ws + 4 * p * TL_LD + 16 * u + (c >> 3);  // column c + 16t: word + 2t, element c & 7
+  const int sh = 4 * nib_pos(c & 7);
   uint32_t wd[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {      // rows 4p + 2h, 4p + 2h + 1 -> words 2h, 2h + 1
+  for (int h = 0; h < 2; ++h) {  // rows 4p + 2h, 4p + 2h + 1 -> words 2h, 2h + 1
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-      const int col = g * 128 + c + 16 * t;
-      const int r = rb * 16 + 4 * p + 2 * h;
-      const uint32_t v = nib(r, col) | (nib(r + 1, col) << 16);
-      wd[2 * h + (t >> 2)] |= v << (4 * (t & 3));
+      const uint32_t lo = (src[2 * h * TL_LD + 2 * t] >> sh) & 0xFu, hi = (src[(2 * h + 1) * TL_LD + 2 * t] >> sh) & 0xFu;
+      wd[2 * h + (t >> 2)] |= (lo | (hi << 16)) << (4 * (t & 3));
     }
   }
-  qt[idx] = make_uint4(wd[0], wd[1], wd[2], wd[3]);
+  qt[((size_t)rb * G + g0 + u) * 64 + l] = make_uint4(wd[0], wd[1], wd[2], wd[3]);
 }
 
 // One 1 KB unit (16 rows x one 128-group) of the tiled matrix, dequantised and dotted with x:
@@ -279,8 +283,7 @@ extern "C" {
 
 int fl_tile_int4(const uint32_t* q, uint32_t* qt, int32_t n, int32_t k, void* stream) {
   if (!q || !qt || n <= 0 || k <= 0 || (n % 16) != 0 || (k % FL_GROUP) != 0) return FL_E_ARG;
-  const int64_t chunks = (int64_t)(n / 16) * (k / 128) * 64;
-  const int64_t blocks = (chunks + 255) / 256;
+  const int64_t blocks = (int64_t)(n / 16) * ((k / 128 + 3) / 4);
   if (blocks > 0x7FFFFFFF) return FL_E_ARG;
   hipLaunchKernelGGL(k_tile_int4, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), q,
                      reinterpret_cast<uint4*>(qt), n, k);

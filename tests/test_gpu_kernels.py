@@ -296,3 +296,58 @@ def test_tiled_gemv_vs_fp64(dev, n, k):
     yr = gemv_int4(q, sz, x.to(dev)).cpu()
     log(f"  bf16 mismatch vs fp64-rounded {mism:.2e}, vs row-layout GEMV {(y != yr).float().mean().item():.2e}")
     assert mism < 2e-3
+
+
+@pytest.mark.parametrize("kind", ["scales", "offset", "constant", "tiny", "inf"])
+def test_quantize_wide_range(dev, kind):
+    """k_quantize divides by a reciprocal and a correction where nothing can overflow and by a true
+    division elsewhere: groups across the bf16 range (both paths within one wave's rows), large offsets,
+    constant and subnormal groups, and groups holding an infinity, against the same steps in
+    torch (each a bf16 operation). Rows that do not fill a workgroup."""
+    from flint_amd.quantize import quantize_int4, unpack_q, unpack_sz
+    g = torch.Generator(device=dev).manual_seed(31)
+    n, k = 173, 640
+    w = torch.randn(n, k, generator=g, device=dev)
+    if kind == "scales":
+        w *= torch.exp2(torch.randint(-100, 120, (n, 1), generator=g, device=dev).float())
+    elif kind == "offset":
+        w = w * 1e-3 + 1000.0 * torch.randn(n, k // 128, generator=g, device=dev).repeat_interleave(128, 1)
+    elif kind == "constant":
+        w = torch.randn(n, k // 128, generator=g, device=dev).repeat_interleave(128, 1)
+    elif kind == "tiny":
+        w *= 2.0 ** -130
+    elif kind == "inf":
+        w[::3, 77] = float("inf")
+    w = w.to(torch.bfloat16).contiguous()
+    x = w.view(-1, 128)
+    mx, mn = x.amax(1, keepdim=True), x.amin(1, keepdim=True)
+    s = (mx - mn).clamp(min=1e-6) / 15
+    z = mn + s * 8
+    t = ((x - (z - s * 8)) / s).round().clamp(0, 15)
+    fine = torch.isfinite(t).all(1).view(n, -1)  # torch's int32 of a NaN is undefined
+    q, sz = quantize_int4(w)
+    got = unpack_q(q).view(n, -1, 128)
+    assert torch.equal(got[fine], t.nan_to_num(0).to(torch.int32).view(n, -1, 128)[fine])
+    gs, gz = unpack_sz(sz)
+    assert torch.equal(gs[fine].view(torch.int16), s.view(n, -1)[fine].view(torch.int16))
+    assert torch.equal(gz[fine].view(torch.int16), z.view(n, -1)[fine].view(torch.int16))
+    assert bool(fine.all()) == (kind != "inf")
+
+
+@pytest.mark.parametrize("n,k", [(16, 128), (32, 256), (48, 640), (16, 16384), (160, 1152)])
+def test_tile_layout(dev, n, k):
+    """fl_tile_int4 at group counts that do and do not fill its workgroups of four, against the layout
+    as the header states it."""
+    from flint_amd.quantize import tile_int4, unpack_q
+    q = torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 8), generator=torch.Generator().manual_seed(n + k), dtype=torch.int64)
+    q = q.to(torch.int32)
+    v = unpack_q(q).view(n // 16, 16, k // 128, 128).to(torch.int64)
+    want = torch.zeros(n // 16, k // 128, 64, 4, dtype=torch.int64)
+    for l in range(64):
+        p, c = (l // 4) % 4, 4 * (l // 16) + l % 4
+        for half in range(2):
+            for t in range(8):
+                pair = v[:, 4 * p + 2 * half, :, c + 16 * t] | v[:, 4 * p + 2 * half + 1, :, c + 16 * t] << 16
+                want[:, :, l, 2 * half + t // 4] |= pair << (4 * (t % 4))
+    got = tile_int4(q.to(dev)).cpu().view(n // 16, k // 128, 64, 4).to(torch.int64) & 0xFFFFFFFF
+    assert torch.equal(got, want)

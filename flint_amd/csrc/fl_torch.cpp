@@ -178,6 +178,50 @@ torch::Tensor int4_linear(torch::Tensor x, torch::Tensor q, torch::Tensor sz, in
   return y;
 }
 
+// The module's forward in one call, for the arguments it can take as they are; None for any other
+// (another dtype or device, strides, a wrong inner dimension): the caller's general path decides
+// those. One row runs the GEMV, up to 32 the GEMM, more the GEMM over rows with a workspace of
+// torch's. From Python the same steps (checks, allocation, ctypes) cost 14 us a call, more than
+// the kernels of one token; here about 5.
+pybind11::object linear_fast(const torch::Tensor& x, const torch::Tensor& q, const torch::Tensor& sz, int64_t stream) {
+  auto plain = [](const torch::Tensor& t, torch::ScalarType dt) {
+    return t.is_cuda() && t.scalar_type() == dt && t.layout() == torch::kStrided && t.is_contiguous();
+  };
+  if (!plain(x, torch::kBFloat16) || !plain(q, torch::kInt32) || !plain(sz, torch::kInt32) || x.dim() < 1 ||
+      q.dim() != 2 || sz.dim() != 2 || sz.size(0) != q.size(0) || sz.size(1) * 16 != q.size(1) ||
+      x.size(-1) != q.size(1) * 8 || x.numel() == 0 || q.numel() == 0)
+    return pybind11::none();
+  const int64_t n = q.size(0), k = q.size(1) * 8, m = x.numel() / k;
+  if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX) return pybind11::none();
+  int64_t ws_bytes = 0;
+  if (m > FL_MAX_VERIFY && fl_gemm_rows_workspace((int32_t)m, (int32_t)n, (int32_t)k, &ws_bytes) != FL_OK)
+    return pybind11::none();
+  torch::Tensor y;
+  int rc;
+  {
+    pybind11::gil_scoped_release nogil;  // a launch may wait for room in the queue
+    auto sizes = x.sizes().vec();
+    sizes.back() = n;
+    y = torch::empty(sizes, x.options().requires_grad(false));
+    auto* xp = reinterpret_cast<const uint16_t*>(x.data_ptr());
+    auto* yp = reinterpret_cast<uint16_t*>(y.data_ptr());
+    auto* qp = reinterpret_cast<const uint32_t*>(q.data_ptr());
+    auto* sp = reinterpret_cast<const uint32_t*>(sz.data_ptr());
+    if (m == 1) {
+      rc = fl_gemv_int4(qp, sp, xp, yp, (int32_t)n, (int32_t)k, stream_of(stream));
+    } else if (m <= FL_MAX_VERIFY) {
+      rc = fl_gemm_int4(qp, sp, xp, yp, (int32_t)m, (int32_t)n, (int32_t)k, stream_of(stream));
+    } else {
+      torch::Tensor ws;
+      if (ws_bytes > 0) ws = torch::empty({ws_bytes / 4}, x.options().dtype(torch::kFloat32).requires_grad(false));
+      rc = fl_gemm_rows_int4(qp, sp, xp, yp, ws_bytes > 0 ? ws.data_ptr<float>() : nullptr, (int32_t)m, (int32_t)n,
+                             (int32_t)k, stream_of(stream));
+    }
+  }
+  if (rc != FL_OK) return pybind11::none();  // the general path raises it
+  return pybind11::cast(y);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -191,5 +235,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def("verify", &Engine::verify)
       .def("check", &Engine::check);
   m.def("int4_linear", &int4_linear);
+  m.def("linear_fast", &linear_fast);
   m.def("version", []() { return fl_version(); });
 }

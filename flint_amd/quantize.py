@@ -5,11 +5,22 @@ Mirrors reference engine/quantize.py:359-525 (prepare_int4_weight_and_scales_and
 linear_forward_int4, WeightOnlyInt4Linear): same groupsize (128), same quantised values,
 same dequantised bf16 values; the packed layout is this library's own (see include/flint_amd.h).
 """
+import os
+
 import torch
 
 from . import _lib
 
 GROUP = _lib.GROUP
+
+# the whole forward of WeightOnlyInt4Linear as one call of the torch extension, over the library
+# beside it (not over another one that FLINT_AMD_LIB names)
+_linear_fast = None
+if "FLINT_AMD_LIB" not in os.environ:
+    try:
+        from ._torch_ops import linear_fast as _linear_fast
+    except ImportError:
+        pass
 
 
 def _check_dev(t, dtype, name):
@@ -170,6 +181,11 @@ class WeightOnlyInt4Linear(torch.nn.Module):
         return m
 
     def forward(self, x):
+        if _linear_fast is not None and type(x) is torch.Tensor and x.is_cuda:
+            y = _linear_fast(x, self.weight, self.scales_and_zeros,
+                             torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+            if y is not None:
+                return y
         shape = x.shape
         x2 = x.reshape(-1, shape[-1]).to(torch.bfloat16).contiguous()
         if x2.shape[0] == 1:

@@ -351,3 +351,40 @@ def test_tile_layout(dev, n, k):
                 want[:, :, l, 2 * half + t // 4] |= pair << (4 * (t % 4))
     got = tile_int4(q.to(dev)).cpu().view(n // 16, k // 128, 64, 4).to(torch.int64) & 0xFFFFFFFF
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("shape", [(1,), (1, 1), (5,), (2, 16), (33,), (4, 100)])
+def test_linear_module_call(dev, shape):
+    """WeightOnlyInt4Linear's single-call forward gives the general path's bits, on another stream and
+    under graph capture too; a strided input, fp32, a subclass and an empty batch take the general path."""
+    from flint_amd import quantize as Q
+    n, k = 2570, 640
+    mod = Q.WeightOnlyInt4Linear.from_float(_weights(n, k, 41).to(dev))
+    x = torch.randn(*shape, k, generator=torch.Generator().manual_seed(42)).to(torch.bfloat16).to(dev)
+    assert Q._linear_fast is not None
+    x2 = x.view(-1, k)
+    want = (Q.gemv_int4(mod.weight, mod.scales_and_zeros, x2[0]).view(1, n) if x2.shape[0] == 1
+            else Q.gemm_int4(mod.weight, mod.scales_and_zeros, x2)).view(*shape, n)
+    assert torch.equal(mod(x), want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        y = mod(x)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(y, want)
+    wide = torch.zeros(*shape, k + 8, dtype=torch.bfloat16, device=dev)
+    wide[..., :k] = x
+    assert torch.equal(mod(wide[..., :k]), want) and torch.equal(mod(x.float()), want)
+    assert torch.equal(mod(torch.nn.Parameter(x, requires_grad=False)), want)
+    assert mod(x[:0]).shape == (0, *shape[1:], n)
+    with pytest.raises(ValueError):
+        mod(x.cpu())
+    g = torch.cuda.CUDAGraph()
+    xs = x.clone()
+    with torch.cuda.graph(g):
+        y = mod(xs)
+    for i in range(3):
+        xs.copy_(x * (i + 1))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, mod(x * (i + 1)))

@@ -10,13 +10,12 @@
 // consecutive weight rows of one activation row: RoPE pairs and gate/up pairs (adjacent packed
 // rows) meet in one lane.
 //
-// What bounds it: matrix-core time plus what does not hide under it. 2048 x 16384 x 2560 takes 228 us
-// (753 TFLOP/s; 64 launches of the 32-row kernel took 1489). In timing builds of it the MFMAs and
-// barriers alone took 158 us, the dequantisation alone about 100: a v_dot2_f32_bf16 of the dequantisation
-// runs on the matrix pipe itself (measured: beside a wave that issues MFMAs it gets next to no
-// slots, where a v_fma_f32 keeps its rate), and other vector instructions issue at 0.6 of their rate beside 16x16 MFMAs.
-// Measured and not taken: the next group's dequantisation interleaved with the MFMAs by hand (258 us), 32x32x16
-// MFMAs (250; they leave the vector ALUs free, but need twice the LDS reads per wave).
+// What bounds it: matrix-core time plus vector time, which hardly overlap here. 2048 x 16384 x 2560 in
+// 128 x 128 tiles took 228 us (64 launches of the former 32-row kernel 1489); in timing builds the MFMAs
+// and barriers alone took 158 us, the dequantisation alone about 100. A v_dot2_f32_bf16 of the dequantisation
+// runs on the matrix pipe itself (measured: beside a wave that issues MFMAs it gets next to no slots, where a
+// v_fma_f32 keeps its rate), and other vector instructions issue at 0.6 of their rate beside 16x16 MFMAs.
+// Calls of many tiles take k_gemm_big below instead (195 us).
 //
 // The ways are for calls of few tiles, where a group's memory latency, not its work, is what a step
 // costs: 32 rows x 16384 x 2560 (256 tiles) takes 20 steps of one way or 5 of four, 64 rows 19 and
@@ -24,6 +23,7 @@
 // Two groups requested ahead instead of one (WD, XD) gain 7-10% with one way on the tiled layout (2048 x
 // 16384 x 2560 222 -> 206 us), and lose with more ways (the registers cost a workgroup per CU).
 #pragma once
+#include <algorithm>
 #include <type_traits>
 #include "fl_common.h"
 
@@ -34,12 +34,30 @@ struct GemmArgs {
   int m, n, k;
   int nblk, mblk;      // tiles along N and M
   int splits, gps;     // K cut into `splits` parts of gps 128-groups
+  int mper;            // tiles along M of one block of the launch order
+
+  // tiles of bn x bm; X blocks of about 3 MB
+  void tile(int bn, int bm) {
+    nblk = (n + bn - 1) / bn;
+    mblk = (m + bm - 1) / bm;
+    const long rows = std::max(1L, (3L << 20) / (2L * gps * FL_GROUP));
+    mper = (int)std::max(1L, std::min<long>(mblk, rows / bm));
+  }
 };
 
-// Workgroups: the tiles of one (weight block, K part) along M run next to each other on one XCD
-// (blockIdx % 8 picks the XCD), so a weight tile comes from HBM once, into one L2.
+// Workgroups: blockIdx % 8 picks the XCD. Along M the tiles are taken in blocks of `mper`, small
+// enough that a block's X stays in an XCD's L2 (4 MB); within a block, the tiles of one (weight block, K
+// part) run next to each other on one XCD, so a weight tile comes from HBM once per block, into one L2.
 inline unsigned gemm_grid(const GemmArgs& a) {
   return 8u * (unsigned)((a.nblk * a.splits + 7) / 8) * (unsigned)a.mblk;
+}
+__device__ __forceinline__ bool gemm_tile(const GemmArgs& a, int& u, int& mb) {
+  const int units = (a.nblk * a.splits + 7) >> 3;  // weight blocks x K parts of an XCD
+  const int j = (int)(blockIdx.x >> 3), blk = j / (units * a.mper), jj = j - blk * units * a.mper;
+  const int mper = min(a.mper, a.mblk - blk * a.mper);
+  u = (jj / mper) * 8 + (int)(blockIdx.x & 7);
+  mb = blk * a.mper + jj % mper;
+  return u < a.nblk * a.splits;
 }
 
 // Epi(n, m, v, split): v[i] = the (partial) sum of weight row n + i and activation row m; n is a
@@ -55,10 +73,10 @@ __global__ __launch_bounds__(64 * NW * KW, NW * KW > 8 ? 4 : 2) void k_gemm_rows
   const int wv0 = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int wave = wv0 % NW, way = wv0 / NW, tid = wave * 64 + lane;  // within the way
   unsigned char (*const xs)[BM * 256] = reinterpret_cast<unsigned char (*)[BM * 256]>(smem + way * (2 * BM * 256));
-  const int j = (int)(blockIdx.x >> 3), u = (j / a.mblk) * 8 + (int)(blockIdx.x & 7);
-  if (u >= a.nblk * a.splits) return;
+  int u, mb;
+  if (!gemm_tile(a, u, mb)) return;
   const int split = u % a.splits, G = a.k >> 7;
-  const int m0 = (j % a.mblk) * BM, n0 = (u / a.splits) * BN + wave * (16 * NB);
+  const int m0 = mb * BM, n0 = (u / a.splits) * BN + wave * (16 * NB);
   // this way's groups; every way passes the same number of barriers
   const int gs0 = split * a.gps, gs1 = min(G, gs0 + a.gps), per = (gs1 - gs0 + KW - 1) / KW;
   const int g0 = gs0 + way * per, g1 = min(gs1, g0 + per);
@@ -235,4 +253,181 @@ __global__ __launch_bounds__(64 * NW * KW, NW * KW > 8 ? 4 : 2) void k_gemm_rows
   for (int b = 0; b < NB; ++b)
 #pragma unroll
     for (int i = 0; i < MB; ++i) epi(n0 + 16 * b + 4 * c, m0 + 16 * i + r, acc[b][i], split);
+}
+
+typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
+
+// The same product for calls of many tiles: BN = 32 NW weight rows x BM = 32 TB activation rows per
+// workgroup, on 32x32x16 MFMAs. A wave dequantises the operand of the next MFMA step (32 rows x 16 k)
+// between the MFMAs of the current one, and reads its X fragments a step ahead, in that order
+// (sched_barrier): beside 32x32 MFMAs the vector ALUs keep 0.9 of their rate (0.6 beside 16x16 ones), and a
+// step's own VALU work then hides under its MFMAs. Both layouts run the 4x4x4 MFMA form of the dequantisation
+// (unit_dq_t's steps; v_dot2 would take matrix-pipe time): a lane needs one column of four rows per step. The
+// tiled layout holds that; from the row layout a lane loads the word it needs of each of its four rows
+// (4-byte loads) and pairs their halves, and takes columns 8 apart in a step, which X in LDS follows.
+// 1024 x 16384 x 2560: tiled 101 us, row 108 (k_gemm_rows with 128 x 128 tiles: 115, 128); 512: 53, 56 (57, 67).
+// What is left (timing builds of the tiled form, 118 us there): the MFMAs alone 63 us, which is 1.5
+// PFLOP/s, the rate that this card holds on any product; without the dequantisation 82; without storing X to LDS 99.
+template <bool TILED, int NW, int TB, class Epi>
+__global__ __launch_bounds__(64 * NW, 2) void k_gemm_big(GemmArgs a, Epi epi) {
+  constexpr int BN = 32 * NW, BM = 32 * TB, RP = 4 * NW, XI = BM / RP;
+  __shared__ __align__(16) unsigned char xs[2][BM * 256];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, c = lane >> 4, r32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int u, mb;
+  if (!gemm_tile(a, u, mb)) return;
+  const int split = u % a.splits, G = a.k >> 7;
+  const int m0 = mb * BM, n0 = (u / a.splits) * BN + wave * 32;
+  const int g0 = split * a.gps, g1 = min(G, g0 + a.gps);
+  const auto xr = buf_rsrc(a.x, (uint32_t)a.m * (uint32_t)a.k * 2u);
+  const auto wr = buf_rsrc(a.q, (uint32_t)a.n * (uint32_t)(a.k >> 1));
+  const auto sr = buf_rsrc(a.sz, (uint32_t)a.n * (uint32_t)G * 4u);
+  const uint32_t xoff = ((uint32_t)(m0 + (tid >> 4)) * (uint32_t)a.k + (uint32_t)(tid & 15) * 8u) * 2u;
+  const uint32_t xstep = (uint32_t)a.k * (2u * RP);
+  const uint32_t kb = (uint32_t)(a.k >> 1);  // bytes of a weight row
+  const uint32_t woff = TILED ? (uint32_t)((n0 >> 4) + (c & 1)) * (uint32_t)G * 1024u + (uint32_t)((c & 2) * 16 + r) * 16u
+                              : (uint32_t)(n0 + 16 * (c & 1) + 4 * ((lane >> 2) & 3)) * kb + (uint32_t)(h * 8 + (lane & 3)) * 4u;
+  const uint32_t soff = (uint32_t)(n0 + r32) * (uint32_t)G * 4u;
+  uint4 xv[XI], wv[2];
+  uint32_t sv;
+  auto load_w = [&](int g) {
+    const bool in = g < g1;
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      if constexpr (TILED) {
+        wv[l] = buf_ld128(wr, in ? woff + (uint32_t)l * 256u + (uint32_t)g * 1024u : 0xFFFFFFF0u);
+      } else {
+        uint32_t t[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          t[e] = buf_ld32(wr, in ? woff + (uint32_t)e * kb + (uint32_t)l * 16u + (uint32_t)g * 64u : 0xFFFFFFF0u);
+        wv[l] = make_uint4(t[0], t[1], t[2], t[3]);
+      }
+    }
+    sv = buf_ld32(sr, in ? soff + (uint32_t)g * 4u : 0xFFFFFFF0u);
+  };
+  auto load_x = [&](int g) {
+    const bool in = g < g1;
+#pragma unroll
+    for (int i = 0; i < XI; ++i) xv[i] = buf_ld128(xr, in ? xoff + (uint32_t)i * xstep + (uint32_t)g * 256u : 0xFFFFFFF0u);
+  };
+  const int st = tid >> 4, un = tid & 15;
+  auto store_x = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+      unsigned char* row = xs[buf] + (st + i * RP) * 256;
+      const int sw = (st + i * RP) & 15;
+      if constexpr (TILED) {
+        const int s0 = (un & 12) + 2 * (un & 1), half = (un >> 1) & 1;
+        *reinterpret_cast<uint2*>(row + ((s0 ^ sw) * 16) + half * 8) = make_uint2(xv[i].x, xv[i].y);
+        *reinterpret_cast<uint2*>(row + (((s0 + 1) ^ sw) * 16) + half * 8) = make_uint2(xv[i].z, xv[i].w);
+      } else {
+        const uint32_t v4[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+#pragma unroll
+        for (int p = 0; p < 4; ++p) *reinterpret_cast<uint32_t*>(row + ((((un & 12) + p) ^ sw) * 16) + (un & 3) * 4) = v4[p];
+      }
+    }
+  };
+  const MxLane mx = mx_lane();
+  const fl_s16x4 ai = mx_s4(0x3F803F80u & mx.mlo, 0x3F803F80u & mx.mhi);
+  uint32_t v[2][4];
+  fl_s16x4 bs;
+  fl_f32x4 c1, c2;
+  auto take = [&]() {  // the group's words and constants from the prefetch registers
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      const uint4 w = wv[l];
+      if constexpr (TILED) {
+        v[l][0] = w.x, v[l][1] = w.y, v[l][2] = w.z, v[l][3] = w.w;
+      } else {
+        v[l][0] = __builtin_amdgcn_perm(w.y, w.x, 0x05040100u);
+        v[l][1] = __builtin_amdgcn_perm(w.y, w.x, 0x07060302u);
+        v[l][2] = __builtin_amdgcn_perm(w.w, w.z, 0x05040100u);
+        v[l][3] = __builtin_amdgcn_perm(w.w, w.z, 0x07060302u);
+      }
+    }
+    const uint32_t sb = sv & 0xFFFFu, sp = sb | (sb << 16);
+    bs = mx_s4(sp & mx.mlo, sp & mx.mhi);
+    const float c1v = -136.0f * bf2f(sb), zv = bf2f(sv >> 16);
+    c1 = fl_f32x4{c1v, c1v, c1v, c1v};
+    c2 = fl_f32x4{zv, zv, zv, zv};
+  };
+  fl_f32x4 d[2];
+  uint32_t p[2][2];
+  auto dq1 = [&](int l, int tp) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int t = TILED ? 2 * tp + e : tp + 4 * e;
+      const uint32_t lo = v[l][t >> 2] >> (4 * (t & 3)), hi = v[l][2 + (t >> 2)] >> (4 * (t & 3));
+      d[e] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(mx_s4((lo & mx.mask) | mx.magic, (hi & mx.mask) | mx.magic), bs, c1, 0, 0, 0);
+    }
+  };
+  auto dq2 = [&]() {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      p[e][0] = pack_bf16x2(d[e][0], d[e][1]);
+      p[e][1] = pack_bf16x2(d[e][2], d[e][3]);
+    }
+  };
+  auto dq3 = [&]() {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) d[e] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ai, mx_s4(p[e][0], p[e][1]), c2, 0, 0, 0);
+  };
+  auto dq4 = [&]() {
+    return TILED ? make_uint4(pack_bf16x2(d[0][0], d[0][1]), pack_bf16x2(d[0][2], d[0][3]), pack_bf16x2(d[1][0], d[1][1]), pack_bf16x2(d[1][2], d[1][3]))
+                 : make_uint4(pack_bf16x2(d[0][0], d[1][0]), pack_bf16x2(d[0][1], d[1][1]), pack_bf16x2(d[0][2], d[1][2]), pack_bf16x2(d[0][3], d[1][3]));
+  };
+  fl_f32x16 acc[TB];
+#pragma unroll
+  for (int i = 0; i < TB; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+  const unsigned char* xb = xs[0] + r32 * 256;
+  auto rd = [&](int buf, int s, int i) {  // X fragment of step s = 4l + tp, token tile i
+    const int l = s >> 2, tp = s & 3, slot = TILED ? 4 * tp + 2 * h + l : 4 * (2 * h + l) + tp;
+    return *reinterpret_cast<const uint4*>(xb + buf * (BM * 256) + i * 8192 + ((slot ^ r) * 16));
+  };
+  uint4 wq, xf[TB];
+  load_w(g0);
+  load_x(g0);
+  store_x(0);
+  take();
+  load_w(g0 + 1);
+  dq1(0, 0); dq2(); dq3(); wq = dq4();
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < TB; ++i) xf[i] = rd(0, 0, i);
+  for (int g = g0; g < g1; ++g) {
+    const int buf = (g - g0) & 1;
+    load_x(g + 1);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      if (s == 6) store_x(buf ^ 1);
+      if (s == 7) {
+        take();          // the next group's words
+        load_w(g + 2);
+        lds_barrier();   // its X is in LDS; every wave has read this group's
+      }
+      uint4 xn[TB], wn;
+#pragma unroll
+      for (int i = 0; i < TB; ++i) {
+        __builtin_amdgcn_sched_barrier(0);
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fl_bf16x8, wq), __builtin_bit_cast(fl_bf16x8, xf[i]), acc[i], 0, 0, 0);
+        xn[i] = s < 7 ? rd(buf, s + 1, i) : rd(buf ^ 1, 0, i);
+        if (i * 4 / TB == 0 && (i == 0 || TB < 4)) dq1(s < 7 ? (s + 1) >> 2 : 0, (s + 1) & 3);
+        if (i == TB / 4) { if (TB >= 4) dq2(); }
+        if (i == TB / 2) { if (TB < 4) dq2(); dq3(); }
+        if (i == TB - 1) wn = dq4();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < TB; ++i) xf[i] = xn[i];
+      wq = wn;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TB; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      epi(n0 + 8 * e + 4 * h, m0 + 32 * i + r32, fl_f32x4{acc[i][4 * e], acc[i][4 * e + 1], acc[i][4 * e + 2], acc[i][4 * e + 3]}, split);
 }

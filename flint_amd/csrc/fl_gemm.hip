@@ -42,8 +42,9 @@ __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ p, 
   out(nn, mm, v, 0);
 }
 
-// How a call of m rows runs. 128 x 128 tiles where they fill the chip (256 CUs, two workgroups each):
-// 512 / 2048 rows x 16384 x 2560 took 60 / 235 us, 64 x 64 tiles 75 / 290. Else 64 x 64 tiles:
+// How a call of m rows runs. Tiles of 128 rows x 256 weight rows (k_gemm_big, one workgroup per CU) where
+// they nearly fill the 256 CUs: 512 / 2048 rows x 16384 x 2560 took 56 / 195 us, 64 x 64 tiles 75 / 290.
+// Else 64 x 64 tiles:
 // - up to 64 rows: four ways, and K cut until there are about 192 workgroups of at least four
 //   128-groups: 64 x 16384 x 2560 took 18 us with one way and 15 with four, 64 x 2560 x 8192 (40 tiles)
 //   36 us uncut and 12 in four parts;
@@ -58,7 +59,7 @@ struct Plan {
 Plan plan_rows(int m, int n, int k) {
   const int G = k / FL_GROUP;
   Plan p{true, 1, 1, G};
-  if ((int64_t)((m + 127) / 128) * ((n + 127) / 128) >= 256) return p;
+  if ((int64_t)((m + 127) / 128) * ((n + 255) / 256) >= 224) return p;
   p.big = false;
   const int64_t tiles = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
   int64_t s = 768 / tiles, most = 8;
@@ -78,8 +79,7 @@ Plan plan_rows(int m, int n, int k) {
 
 template <int NW, int KW, int NB, int MB, class Epi>
 void launch(GemmArgs a, Epi epi, hipStream_t s) {
-  a.nblk = (a.n + 16 * NW * NB - 1) / (16 * NW * NB);
-  a.mblk = (a.m + 16 * MB - 1) / (16 * MB);
+  a.tile(16 * NW * NB, 16 * MB);
   hipLaunchKernelGGL((k_gemm_rows<false, NW, KW, NB, MB, 1, 1, Epi>), dim3(gemm_grid(a)), dim3(64 * NW * KW), 0, s, a, epi);
 }
 template <class Epi>
@@ -109,7 +109,7 @@ int fl_gemm_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint1
   if (m < 1 || m > FL_MAX_VERIFY) return FL_E_M;
   if ((int64_t)n * (k / 2) > 0xFFFFFFFFll || (int64_t)m * k * 2 > 0xFFFFFFFFll) return FL_E_ARG;
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const GemmArgs a{q, sz, x, m, n, k, 0, 0, 1, k / FL_GROUP};
+  const GemmArgs a{q, sz, x, m, n, k, 0, 0, 1, k / FL_GROUP, 0};
   const EpiBf16 epi = out_bf16(y, m, n);
   // One workgroup per 64 weight rows (four ways) where that gives at least 192, else one per 16 rows
   // with as many ways as the LDS holds: 32 rows x 16384 x 2560 12 us (four ways; 23 in the former
@@ -149,9 +149,11 @@ int fl_gemm_rows_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, 
     const int rows = std::min(ROWS_PER_LAUNCH, m - r0);
     const Plan p = plan_rows(rows, n, k);
     const EpiBf16 epi = out_bf16(y + (size_t)r0 * n, rows, n);
-    const GemmArgs a{q, sz, x + (size_t)r0 * k, rows, n, k, 0, 0, p.splits, p.gps};
+    const GemmArgs a{q, sz, x + (size_t)r0 * k, rows, n, k, 0, 0, p.splits, p.gps, 0};
     if (p.big) {
-      launch<4, 1, 2, 8>(a, epi, s);
+      GemmArgs b = a;
+      b.tile(256, 128);
+      hipLaunchKernelGGL((k_gemm_big<false, 8, 4, EpiBf16>), dim3(gemm_grid(b)), dim3(512), 0, s, b, epi);
     } else if (p.splits == 1) {
       launch_small(p.ways, a, epi, s);
     } else {

@@ -6,7 +6,7 @@
 //   residual + RMSNorm -> gate/up GEMM (SwiGLU in its epilogue) -> down GEMM -> residual + RMSNorm,
 // the O and down GEMMs cut along K into fp32 part sums that the residual kernel adds in order. After
 // the last pass the LM head and argmax of the last token.
-// At 512 tokens of flint-3b a layer takes 170 us (of which the GEMMs: QKV 24, O 20, gate/up 57, down 44;
+// At 512 tokens of flint-3b a layer takes 157 us (of which the GEMMs: QKV 24, O 19, gate/up 50, down 36;
 // attention 17, the two norms 13), against 1336 in sixteen k_verify launches; 40 tokens take 64 us a
 // layer (launches and latency) against 120, and up to 32 they take the one k_verify launch (n = 16:
 // 46 us a layer against 61; n = 32: 80 against 62, but at 12000 cached keys 125 against 150).
@@ -16,8 +16,6 @@
 #include <string.h>
 
 namespace {
-
-typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int PF_TOKENS = 1024;  // tokens of a pass at most: 512 per pass cost 13.6 us a token, 1024 10.9
 constexpr int PF_NT = 256;
@@ -414,38 +412,42 @@ PfWs pf_layout(const fl_model_desc& d, int T, uint8_t* base) {
 
 template <int NW, int KW, int MB, class Epi>
 void pf_launch(GemmArgs a, Epi epi, hipStream_t s) {
-  a.nblk = (a.n + 16 * NW - 1) / (16 * NW);
-  a.mblk = (a.m + 16 * MB - 1) / (16 * MB);
+  a.tile(16 * NW, 16 * MB);
   constexpr int D = KW == 1 ? 2 : 1;  // groups requested ahead
   hipLaunchKernelGGL((k_gemm_rows<true, NW, KW, 1, MB, D, D, Epi>), dim3(gemm_grid(a)), dim3(64 * NW * KW), 0, s, a, epi);
 }
 
-// One GEMM of a pass, in 64 x 64 tiles (four waves a way) or 128 x 128 (eight). `parts`: the epilogue
-// keeps fp32 sums of K parts, which k_pf_norm adds; returns their number. Measured at flint-3b's
-// sizes (us):
-// - up to 256 tiles of 64 four ways, up to 512 two: QKV at 64 / 512 tokens (56 / 448 tiles) 19 / 28 with one
-//   way, 12 / - with four, - / 21 with two; gate/up at 64 (256) 20 and 13, at 100 (512) 24 and 21;
-// - more: tiles of 128 if those are at least 160 (gate/up at 512 tokens 58, 64 x 64 tiles 75), else 64;
-// - parts of 64 x 64 tiles: about ten groups each, four at most, more while they give fewer than 160
-//   workgroups. O at 512 tokens (320 tiles) 18 us in two parts, 17 in four, whose sums cost more to add;
-//   down 41 in four, 47 in two; at 64 tokens O 7 in four, down 11 in four with four ways, 16 with one;
-// - parts of 128 x 128 tiles: two workgroups per CU. At 1024 tokens (160 tiles; 640 of 64) O 27 us in
-//   three parts and 31 in two, down 65 in three and 71 in four.
+// One GEMM of a pass. `parts`: the epilogue keeps fp32 sums of K parts, which k_pf_norm adds;
+// returns their number. Measured at flint-3b's sizes (us, weights from HBM):
+// - tiles of 256 x 128 (k_gemm_big, one workgroup per CU) where they and the parts give at least 160
+//   workgroups: gate/up at 512 / 1024 tokens (256 / 512 tiles) 53 / 101, 57 / 115 in tiles of 128 x 128; down at
+//   512 (40 tiles) 39 in four parts, 42 in tiles of 64 x 64; O at 512 has too few groups for four parts of eight;
+// - else tiles of 64 x 64, up to 256 of them four ways, up to 512 two: QKV at 64 / 512 tokens (56 / 448 tiles)
+//   20 / 27 with one way, 14 / - with four, - / 24 with two; gate/up at 64 (256) 21 and 15; parts of about ten
+//   groups, four at most, more while they give fewer than 160 workgroups: O at 512 (320 tiles) 19 in two parts,
+//   at 64 tokens 8 in four; down at 64 tokens 11 in four with four ways, 16 with one;
+// - tiles of 128 x 128 in between: QKV at 1024 (224 tiles) 39.
 template <class Epi>
 int pf_gemm(const uint32_t* qt, const uint32_t* sz, const uint16_t* x, int T, int n, int k, bool parts, Epi epi,
             hipStream_t s) {
   const int G = k / FL_GROUP;
-  GemmArgs a{qt, sz, x, T, n, k, 0, 0, 1, G};
+  GemmArgs a{qt, sz, x, T, n, k, 0, 0, 1, G, 0};
   const int t64 = ((n + 63) / 64) * ((T + 63) / 64), t128 = ((n + 127) / 128) * ((T + 127) / 128);
-  const bool big = t64 > 512 && t128 >= 160;
-  if (parts) {
-    const int want = big ? 512 / t128 : std::max(G / 10, (160 + t64 - 1) / t64);
-    a.splits = std::max(1, std::min({PF_SPLITS, want, G / 4}));
-    a.gps = (G + a.splits - 1) / a.splits;
+  const int t256 = ((n + 255) / 256) * ((T + 127) / 128);
+  auto cut = [&](int want, int least) {  // K in `want` parts of at least `least` groups
+    const int s = std::max(1, std::min({PF_SPLITS, want, G / least}));
+    a.gps = (G + s - 1) / s;
     a.splits = (G + a.gps - 1) / a.gps;
+  };
+  if (parts) cut(256 / t256, 8);
+  if (t256 * a.splits >= 160) {
+    a.tile(256, 128);
+    hipLaunchKernelGGL((k_gemm_big<true, 8, 4, Epi>), dim3(gemm_grid(a)), dim3(512), 0, s, a, epi);
+    return a.splits;
   }
+  if (parts) cut(std::max(G / 10, (160 + t64 - 1) / t64), 4);
   const int wgs = t64 * a.splits;
-  if (big) pf_launch<8, 1, 8>(a, epi, s);
+  if (!parts && t128 >= 160) pf_launch<8, 1, 8>(a, epi, s);
   else if (wgs <= 256 && a.gps >= 8) pf_launch<4, 4, 4>(a, epi, s);
   else if (wgs <= 512 && a.gps >= 8) pf_launch<4, 2, 4>(a, epi, s);
   else pf_launch<4, 1, 4>(a, epi, s);

@@ -6,10 +6,10 @@
 //   residual + RMSNorm -> gate/up GEMM (SwiGLU in its epilogue) -> down GEMM -> residual + RMSNorm,
 // the O and down GEMMs cut along K into fp32 part sums that the residual kernel adds in order. After
 // the last pass the LM head and argmax of the last token.
-// At 512 tokens of flint-3b a layer takes 157 us (of which the GEMMs: QKV 24, O 19, gate/up 50, down 36;
-// attention 17, the two norms 13), against 1336 in sixteen k_verify launches; 40 tokens take 64 us a
-// layer (launches and latency) against 120, and up to 32 they take the one k_verify launch (n = 16:
-// 46 us a layer against 61; n = 32: 80 against 62, but at 12000 cached keys 125 against 150).
+// At 512 tokens of flint-3b a layer takes 151 us (of which the GEMMs: QKV 24, O 19, gate/up 52, down 38;
+// attention 12, the two norms 13), against 1336 in sixteen k_verify launches; 40 tokens take 64 us a
+// layer (launches and latency) against 120, and up to 16 they take the one k_verify launch (16: 46 us a
+// layer against 62; 24: 71 against 62, at 12000 cached keys 118 against 85).
 #include "fl_gemm.h"
 #include "fl_state.h"
 #include <algorithm>
@@ -20,6 +20,7 @@ namespace {
 constexpr int PF_TOKENS = 1024;  // tokens of a pass at most: 512 per pass cost 13.6 us a token, 1024 10.9
 constexpr int PF_NT = 256;
 constexpr int PF_SPLITS = 4;      // K parts of the O and down GEMMs at most
+constexpr int PF_KEY_PARTS = 16;  // key parts of the attention at most
 constexpr int PF_NORM_MAX = 3;    // 4-value chunks per thread of a row (D <= 3072)
 constexpr int PF_LM_GRID = 512;   // LM-head workgroups
 
@@ -129,37 +130,47 @@ __global__ __launch_bounds__(PF_NT) void k_pf_norm(const float* __restrict__ par
 
 // ---- attention --------------------------------------------------------------------------------------
 // The rows of a KV group are its (token, query head) pairs, token-major: row t * rep + j. A workgroup
-// takes 128 rows of a group (32 per wave) over one part of the keys [0, pos + its last token], in tiles
-// of 64 keys staged in LDS (K rows; V transposed), double-buffered, so a group's K / V rows are read
-// once per 128 rows. Per tile S^T = K Q^T on 32x32x16 MFMAs (lane = row, registers = keys), an online
-// fp32 softmax per lane, and O^T += V^T P^T with P split into three bf16 terms (hi + mid + lo, each
-// product exact, as k_verify's attention): the keys of a 16-key step are taken in the order
-// that the score registers already hold them, so P needs no exchange between lanes.
-constexpr int PA_KEYS = 64;
-constexpr int PA_VLD = 68;  // V^T row pitch (bf16): 34 words spread a wave's 8-byte reads over all banks
+// takes 128 / W rows of a group over one part of the keys [0, pos + its last token], in rounds of 64 W keys
+// staged in LDS (K rows; V transposed), double-buffered, so a group's K / V rows are read once per
+// workgroup. Its four waves are W ways of 4 / W: a way's waves take 32 rows each over the way's 64 keys of
+// every round, and the ways' (max, sum, o) meet in LDS at the end. Two ways by default: a row's keys are a
+// serial chain, and 512 tokens of flint-3b are only 320 workgroups of 64 rows (one way, 160 of 128: 16.8
+// us, two 11.5); one way, which stages each key for twice the rows, where 128-row workgroups fill the
+// chip and the keys are many (1024 tokens behind 4000 / 12000 keys: 403 / 672 us a layer, 418 / 716
+// with two ways; behind none 274 and 267).
+// Per 64 keys S^T = K Q^T on 32x32x16 MFMAs (lane = row, registers = keys), an online fp32 softmax per
+// lane, and O^T += V^T P^T with P split into three bf16 terms (hi + mid + lo, each product exact, as
+// k_verify's attention): the keys of a 16-key step are taken in the order that the score
+// registers already hold them, so P needs no exchange between lanes. Bound by the vector ALUs
+// (about 350 instructions per 64 keys and wave, 1.7x the MFMAs' cycles).
+constexpr int PA_WGS = 512;   // workgroups that cutting the keys into parts may reach
+constexpr int PA_VLD = 68;    // V^T row pitch of a way (bf16): 34 words spread a wave's 8-byte reads over all banks
 struct PaArgs {
   const uint16_t *q, *kc, *vc;  // q [T][NH * 64], kc / vc of this layer
   uint16_t* out;                // [T][NH * 64]
   float* part;                  // with key parts: o [parts][NKV][rows][64], then (m, l) [parts][NKV][rows][2]
   int T, pos, S, nh, nkv, rep;
-  int blocks, parts, kpp;       // 128-row blocks per group; key parts, keys per part (multiple of 64)
+  int blocks, parts, kpp;       // row blocks per group; key parts, keys per part (multiple of 128)
   float sc;                     // attn_scale * log2 e
 };
 
-__global__ __launch_bounds__(256) void k_pf_attn(PaArgs a) {
+template <int W>
+__global__ __launch_bounds__(256, 2) void k_pf_attn(PaArgs a) {
+  constexpr int PA_ROWS = 128 / W, PA_KEYS = 64 * W, WR = 4 / W;  // rows, keys per round; waves of a way
   __shared__ __align__(16) unsigned char ks[2][PA_KEYS * 128];
-  __shared__ __align__(16) uint16_t vt[2][64 * PA_VLD];
+  __shared__ __align__(16) uint16_t vt[2][W * 64 * PA_VLD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hf = lane >> 5;
+  const int sub = wave % WR, way = wave / WR;
   const int g = blockIdx.x % a.nkv, rest = blockIdx.x / a.nkv;
   const int part = rest % a.parts, blk = a.blocks - 1 - rest / a.parts;  // the longest rows first
-  const int R = a.T * a.rep, row0 = blk * 128;
-  const int tlast = min(a.T - 1, (row0 + 127) / a.rep);
+  const int R = a.T * a.rep, row0 = blk * PA_ROWS;
+  const int tlast = min(a.T - 1, (row0 + PA_ROWS - 1) / a.rep);
   const int kb0 = part * a.kpp, kend = min(a.pos + tlast + 1, kb0 + a.kpp);  // keys of this workgroup
-  const int row = row0 + wave * 32 + r, rowc = min(row, R - 1);
+  const int row = row0 + sub * 32 + r, rowc = min(row, R - 1);
   const int t = rowc / a.rep, head = g * a.rep + rowc % a.rep;
-  const int lim = a.pos + t;  // the last key this row sees
-  const int wfirst = a.pos + min(row0 + wave * 32, R - 1) / a.rep;       // ... the wave's first row
-  const int wlast = a.pos + min(row0 + wave * 32 + 31, R - 1) / a.rep;   // ... and its last
+  const int lim = min(a.pos + t, kend - 1);  // the last key this row sees here
+  const int wfirst = min(a.pos + min(row0 + sub * 32, R - 1) / a.rep, kend - 1);  // ... the wave's first row
+  const int wlast = a.pos + min(row0 + sub * 32 + 31, R - 1) / a.rep;             // ... and its last
   const size_t cb = (size_t)g * a.S * 64;
   const auto kr = buf_rsrc(a.kc + cb, (uint32_t)(a.pos + a.T) * 128u);  // keys past the end read as zeros
   const auto vr = buf_rsrc(a.vc + cb, (uint32_t)(a.pos + a.T) * 128u);
@@ -167,26 +178,31 @@ __global__ __launch_bounds__(256) void k_pf_attn(PaArgs a) {
 #pragma unroll
   for (int s = 0; s < 4; ++s)
     qf[s] = *reinterpret_cast<const uint4*>(a.q + ((size_t)t * a.nh + head) * 64 + s * 16 + hf * 8);
-  uint4 kv[2], vv[2];
-  const int c8 = tid & 7, kp = tid >> 3;  // 16-byte chunk; K rows kp, kp + 32; V rows 2 kp, 2 kp + 1
+  uint4 kv[2 * W], vv[2 * W];
+  const int c8 = tid & 7, kp = tid >> 3;  // 16-byte chunk; K rows kp + 32 i; V rows 2 kp, 2 kp + 1 of every way
   auto load = [&](int kb) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < 2 * W; ++i) {
       kv[i] = buf_ld128(kr, (uint32_t)(kb + kp + 32 * i) * 128u + (uint32_t)c8 * 16u);
-      vv[i] = buf_ld128(vr, (uint32_t)(kb + 2 * kp + i) * 128u + (uint32_t)c8 * 16u);
+      vv[i] = buf_ld128(vr, (uint32_t)(kb + 64 * (i >> 1) + 2 * kp + (i & 1)) * 128u + (uint32_t)c8 * 16u);
     }
   };
   auto store = [&](int b) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < 2 * W; ++i) {
       const int key = kp + 32 * i;
       *reinterpret_cast<uint4*>(ks[b] + key * 128 + ((c8 ^ ((key >> 1) & 7)) * 16)) = kv[i];
     }
-    const uint32_t x[4] = {vv[0].x, vv[0].y, vv[0].z, vv[0].w}, y[4] = {vv[1].x, vv[1].y, vv[1].z, vv[1].w};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {  // the two keys of a dim side by side
-      *reinterpret_cast<uint32_t*>(&vt[b][(c8 * 8 + 2 * e) * PA_VLD + 2 * kp]) = __builtin_amdgcn_perm(y[e], x[e], 0x05040100u);
-      *reinterpret_cast<uint32_t*>(&vt[b][(c8 * 8 + 2 * e + 1) * PA_VLD + 2 * kp]) = __builtin_amdgcn_perm(y[e], x[e], 0x07060302u);
+    for (int w = 0; w < W; ++w) {
+      const uint32_t x[4] = {vv[2 * w].x, vv[2 * w].y, vv[2 * w].z, vv[2 * w].w};
+      const uint32_t y[4] = {vv[2 * w + 1].x, vv[2 * w + 1].y, vv[2 * w + 1].z, vv[2 * w + 1].w};
+      uint16_t* v = &vt[b][w * 64 * PA_VLD];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {  // the two keys of a dim side by side
+        *reinterpret_cast<uint32_t*>(v + (c8 * 8 + 2 * e) * PA_VLD + 2 * kp) = __builtin_amdgcn_perm(y[e], x[e], 0x05040100u);
+        *reinterpret_cast<uint32_t*>(v + (c8 * 8 + 2 * e + 1) * PA_VLD + 2 * kp) = __builtin_amdgcn_perm(y[e], x[e], 0x07060302u);
+      }
     }
   };
   fl_f32x16 o[2];
@@ -199,18 +215,18 @@ __global__ __launch_bounds__(256) void k_pf_attn(PaArgs a) {
     load(kb0);
     store(0);
   }
-  for (int kb = kb0; kb < kend; kb += PA_KEYS) {
-    const int b = ((kb - kb0) / PA_KEYS) & 1;
-    const bool more = kb + PA_KEYS < kend;
+  for (int kr0 = kb0; kr0 < kend; kr0 += PA_KEYS) {
+    const int b = ((kr0 - kb0) / PA_KEYS) & 1, kb = kr0 + 64 * way;  // this way's 64 keys
+    const bool more = kr0 + PA_KEYS < kend;
     __syncthreads();
-    if (more) load(kb + PA_KEYS);
-    if (kb <= wlast) {  // wave-uniform: some row of the wave sees a key of this tile
+    if (more) load(kr0 + PA_KEYS);
+    if (kb <= wlast && kb < kend) {  // wave-uniform: some row of the wave sees a key of these
       fl_f32x16 s[2];
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[kt][i] = 0.0f;
-        const int key = kt * 32 + r;
+        const int key = 64 * way + kt * 32 + r;
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
           const uint4 kf = *reinterpret_cast<const uint4*>(ks[b] + key * 128 + (((2 * st + hf) ^ ((key >> 1) & 7)) * 16));
@@ -220,13 +236,13 @@ __global__ __launch_bounds__(256) void k_pf_attn(PaArgs a) {
       }
       // s[kt][i]: key kb + 32 kt + 8 (i / 4) + 4 hf + i % 4 of this lane's row
       float mx = -INFINITY;
-      if (kb + PA_KEYS - 1 > wfirst || kb + PA_KEYS > kend) {  // a tile that crosses a row's last key
+      if (kb + 63 > wfirst) {  // keys past some row's last one
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
             const int key = kb + 32 * kt + 8 * (i >> 2) + 4 * hf + (i & 3);
-            s[kt][i] = key <= lim && key < kend ? s[kt][i] * a.sc : -INFINITY;
+            s[kt][i] = key <= lim ? s[kt][i] * a.sc : -INFINITY;
             mx = fmaxf(mx, s[kt][i]);
           }
       } else {
@@ -271,7 +287,7 @@ __global__ __launch_bounds__(256) void k_pf_attn(PaArgs a) {
         const fl_bf16x8 bl = __builtin_bit_cast(fl_bf16x8, make_uint4(pl[0], pl[1], pl[2], pl[3]));
 #pragma unroll
         for (int d = 0; d < 2; ++d) {
-          const uint16_t* vp = &vt[b][(d * 32 + r) * PA_VLD + 16 * st + 4 * hf];
+          const uint16_t* vp = &vt[b][way * 64 * PA_VLD + (d * 32 + r) * PA_VLD + 16 * st + 4 * hf];
           const uint2 v0 = *reinterpret_cast<const uint2*>(vp), v1 = *reinterpret_cast<const uint2*>(vp + 8);
           const fl_bf16x8 va = __builtin_bit_cast(fl_bf16x8, make_uint4(v0.x, v0.y, v1.x, v1.y));
           o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, bh, o[d], 0, 0, 0);
@@ -281,6 +297,29 @@ __global__ __launch_bounds__(256) void k_pf_attn(PaArgs a) {
       }
     }
     if (more) store(b ^ 1);
+  }
+  if constexpr (W == 2) {  // the second way's (max, sum, o) into the first's, through LDS (K's place)
+    __syncthreads();
+    float* mrg = reinterpret_cast<float*>(&ks[0][0]) + sub * (34 * 64) + lane;
+    static_assert(W == 1 || WR * 34 * 64 * 4 <= sizeof(ks), "the ways' exchange fits K's place");
+    if (way == 1) {
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mrg[(d * 16 + i) * 64] = o[d][i];
+      mrg[32 * 64] = mrun;
+      mrg[33 * 64] = lrun;
+    }
+    __syncthreads();
+    if (way == 1) return;
+    const float m1 = mrg[32 * 64], mm = fmaxf(mrun, m1), mu = mm == -INFINITY ? 0.0f : mm;
+    const float e0 = __builtin_amdgcn_exp2f(mrun - mu), e1 = __builtin_amdgcn_exp2f(m1 - mu);
+    mrun = mm;
+    lrun = lrun * e0 + mrg[33 * 64] * e1;
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[d][i] = o[d][i] * e0 + mrg[(d * 16 + i) * 64] * e1;
   }
   if (row >= R) return;
   if (a.parts == 1) {
@@ -403,8 +442,9 @@ PfWs pf_layout(const fl_model_desc& d, int T, uint8_t* base) {
   w.attn = (uint16_t*)take(row);
   w.act = (uint16_t*)take((size_t)T * d.inter * 2);
   // the GEMMs' part sums; the attention's key parts (o and (m, l) per row) take turns with them
-  const size_t rows = (size_t)T * d.n_head;
-  w.part = (float*)take(std::max((size_t)PF_SPLITS * T * d.dim * 4, (size_t)PF_SPLITS * rows * 66 * 4));
+  // (more than one part only while parts x blocks x groups <= PA_WGS workgroups of 64 rows)
+  const size_t rows = std::min((size_t)PF_KEY_PARTS * T * d.n_head, (size_t)PA_WGS * 64);
+  w.part = (float*)take(std::max((size_t)PF_SPLITS * T * d.dim * 4, rows * 66 * 4));
   w.best = (unsigned long long*)take(PF_LM_GRID * 8);
   w.bytes = at;
   return w;
@@ -469,15 +509,21 @@ void pf_attention(const fl_state* st, const PfWs& w, int l, int T, int pos, hipS
   a.nh = d.n_head;
   a.nkv = d.n_kv_head;
   a.rep = d.n_head / d.n_kv_head;
-  a.blocks = (T * a.rep + 127) / 128;
+  const int b128 = (T * a.rep + 127) / 128;
+  // one way for rows that fill the chip behind many keys: 1024 tokens cost 7 us less a layer with two
+  // over no keys and 0.006 us more per key (12 us at 4000), so the two meet near 1100
+  const bool one_way = b128 * a.nkv >= 256 && pos >= 2048;
+  a.blocks = one_way ? b128 : (T * a.rep + 63) / 64;
   a.sc = d.attn_scale * 1.4426950408889634f;
-  // key parts while there are fewer workgroups than CUs, at least four tiles of keys each
+  // key parts up to PA_WGS workgroups (two per CU), at least 256 keys each: 40 tokens behind
+  // 12000 keys (32 workgroups uncut) 94 us a layer, of which 31 over no keys; at most four parts 157
   const int keys = pos + T;
-  int parts = std::min({PF_SPLITS, st->grid / (a.blocks * a.nkv), keys / (4 * PA_KEYS)});
-  parts = std::max(1, parts);
-  a.kpp = ((keys + parts - 1) / parts + PA_KEYS - 1) / PA_KEYS * PA_KEYS;
+  const int parts = one_way ? 1 : std::max(1, std::min({PF_KEY_PARTS, PA_WGS / (a.blocks * a.nkv), keys / 256}));
+  a.kpp = ((keys + parts - 1) / parts + 127) / 128 * 128;
   a.parts = (keys + a.kpp - 1) / a.kpp;
-  hipLaunchKernelGGL(k_pf_attn, dim3(a.blocks * a.parts * a.nkv), dim3(256), 0, s, a);
+  const dim3 grid(a.blocks * a.parts * a.nkv);
+  if (one_way) hipLaunchKernelGGL(k_pf_attn<1>, grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(k_pf_attn<2>, grid, dim3(256), 0, s, a);
   if (a.parts > 1)
     hipLaunchKernelGGL(k_pf_attn_merge, dim3((a.nkv * T * a.rep + 3) / 4), dim3(256), 0, s, a);
 }

@@ -8,9 +8,9 @@ is prefilled through the speculative-verify kernel, up to 32 tokens per launch.
 """
 import torch
 
-# prompts of more tokens than this run as fl_prefill passes (flint-3b, 40 layers: 40 tokens 2.55 ms in a
-# pass and 4.81 in two verify launches; 32 tokens in one launch 3.2 ms, at 12000 cached keys 5.0 against 6.1)
-PREFILL_MIN = 32
+# prompts of more tokens than this run as fl_prefill passes: up to 16 tokens are one token pass of the verify
+# launch (flint-3b, 40 layers: 16 tokens 1.8 ms against 2.5 in a pass, 24 tokens 2.8 against 2.5)
+PREFILL_MIN = 16
 
 
 def prefill(model, x, input_pos, chunk=32):

@@ -1,6 +1,6 @@
 """Prompts through fl_prefill (GEMM passes over many tokens) against the oracle's batched forward:
 the cache rows that it writes and the logits of the step after it, at the edges of its tiles (64 and
-128 tokens), of its 128-row attention blocks, key parts and passes of 1024 tokens."""
+128 tokens), of its attention's blocks of 64 and 128 rows, key parts and passes of 1024 tokens."""
 import pytest
 import torch
 
@@ -39,7 +39,7 @@ def _check(name, eng, orc, n, pos, seed):
     assert float(row.max() - row[am]) <= 2.0 * float((alt[n - 1] - row).abs().max()) + 2.0 ** -5
 
 
-@pytest.mark.parametrize("n,pos", [(33, 0), (63, 5), (64, 0), (65, 300), (127, 1), (129, 0), (333, 250), (700, 100)])
+@pytest.mark.parametrize("n,pos", [(17, 40), (33, 0), (63, 5), (64, 0), (65, 300), (127, 1), (129, 0), (333, 250), (700, 100)])
 def test_prefill_small(dev, n, pos):
     args, sd, eng, orc = make_pair("small", seed=3)
     eng.setup_caches(1, 1100)
@@ -47,10 +47,16 @@ def test_prefill_small(dev, n, pos):
     _check("small", eng, orc, n, pos, seed=n)
 
 
-@pytest.mark.parametrize("name,n,pos", [("tiny", 1000, 0), ("tiny", 40, 900), ("flint-3b-l1", 100, 2000), ("wide", 90, 7)])
+@pytest.mark.parametrize("name,n,pos", [("tiny", 1000, 0), ("tiny", 40, 900), ("tiny", 20, 1000), ("flint-3b-l1", 100, 2000),
+                                        ("wide", 90, 7), ("42 heads", 840, 2100)])
 def test_prefill_shapes(dev, name, n, pos):
-    """Few KV heads; a short prompt behind many keys (key parts); the 3B layer; the widest rows."""
-    args, sd, eng, orc = make_pair(name, seed=4, weight_device="cuda")
+    """Few KV heads; a short prompt behind many keys (key parts); the 3B layer; the widest rows; enough
+    rows for the large GEMM tiles (2688 weight rows: the last tile is half empty) and, behind enough
+    keys, for the attention's one-way form."""
+    over = {}
+    if name == "42 heads":
+        name, over = "flint-3b-l1", dict(n_head=42, n_local_heads=3, dim=2688, vocab_size=2048)
+    args, sd, eng, orc = make_pair(name, seed=4, weight_device="cuda", **over)
     eng.setup_caches(1, n + pos + 1)
     orc.setup_caches(eng.max_seq_length)
     _check(name, eng, orc, n, pos, seed=n)

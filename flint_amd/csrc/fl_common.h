@@ -529,12 +529,16 @@ __device__ __forceinline__ int select_bin(const int* hist, int k, int* above, in
     const int b0 = 4 * tid;
     const int c0 = hist[b0], c1 = hist[b0 + 1], c2 = hist[b0 + 2], c3 = hist[b0 + 3];
     const int own = c0 + c1 + c2 + c3;
-    int incl = own;  // sum over lanes >= tid
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int t = __shfl_down(incl, o, 64);
-      if (tid + o < 64) incl += t;
-    }
+    // sum over lanes >= tid: within a row of 16 by DPP row_shl (lanes past the row read 0), then the
+    // totals of the rows above (each __shfl_down step instead is an LDS round trip)
+    int incl = own;
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x101, 0xF, 0xF, true);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x102, 0xF, 0xF, true);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x104, 0xF, 0xF, true);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x108, 0xF, 0xF, true);
+    const int r1 = __builtin_amdgcn_readlane(incl, 16), r2 = __builtin_amdgcn_readlane(incl, 32),
+              r3 = __builtin_amdgcn_readlane(incl, 48);
+    incl += tid < 16 ? r1 + r2 + r3 : tid < 32 ? r2 + r3 : tid < 48 ? r3 : 0;
     const int hi = incl - own;  // keys in bins above this lane's four
     if (hi < k && incl >= k) {
       // the highest of the four bins where the running count from the top reaches k

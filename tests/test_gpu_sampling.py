@@ -50,6 +50,35 @@ def test_sample_given_noise_matches_oracle(dev, vocab, t, k):
         assert tok[r] == idx or _near_tie(ratio)
 
 
+@pytest.mark.parametrize("rows,vocab,k", [(1, 1, None), (2, 511, 7), (1, 512, 100), (1, 513, 512), (2, 2049, 600),
+                                          (17, 16384, 3000), (3, 65536, 40), (2, 65536, None)])
+@pytest.mark.parametrize("form", ["ties", "masked", "flat"])
+def test_sample_pivot_bin(dev, rows, vocab, k, form):
+    """The softmax sum is taken from partial sums above the pivot's high byte and from counts of equal
+    values inside it: many equal values, with the pivot among them; rows of -inf but for a few values,
+    so that -inf is the pivot; a row of one value. Chunk edges at multiples of 512, a second launch at
+    row 16."""
+    from flint_amd.generate import sample
+    lg = _rows(vocab, rows, vocab)
+    if form == "ties":
+        lg = np.round(lg * 2) / 2
+    elif form == "masked":
+        keep = np.random.default_rng(vocab).random((rows, vocab)) < 3.0 / vocab
+        keep[:, vocab // 2] = True
+        lg = np.where(keep, lg, np.float32(-np.inf))
+    else:
+        lg = np.full_like(lg, -3.25)
+    lg = lg.astype(np.float32)
+    q = np.stack([exponential_noise(6, 0, vocab, r) for r in range(rows)])
+    tok, pr = sample(torch.from_numpy(lg).to(dev), 0.7, k, noise=torch.from_numpy(q).to(dev), probs=True)
+    tok, pr = tok.cpu().numpy(), pr.cpu().numpy()
+    for r in range(rows):
+        p_o, _ = logits_to_probs(lg[r], 0.7, k)
+        idx, ratio = sample_with_noise(lg[r], q[r], 0.7, k)
+        assert np.all(np.abs(pr[r] - p_o) <= np.maximum(np.abs(p_o), 2.0 ** -126) * 2.0 ** -7 + 1e-45)
+        assert tok[r] == idx or vocab > 1 and _near_tie(ratio)
+
+
 def test_sample_philox_noise_matches_oracle(dev):
     from flint_amd.generate import sample
     vocab, rows = 49152, 8

@@ -48,16 +48,28 @@ struct GemmArgs {
 // Workgroups: blockIdx % 8 picks the XCD. Along M the tiles are taken in blocks of `mper`, small
 // enough that a block's X stays in an XCD's L2 (4 MB); within a block, the tiles of one (weight block, K
 // part) run next to each other on one XCD, so a weight tile comes from HBM once per block, into one L2.
+// The last units % 8 of these are dealt in eight equal runs of tiles instead: 333 x 2570 x 2560 (41 weight
+// blocks of 6 tiles) otherwise gives one XCD 36 of 246 four-way workgroups for its 32 CUs and takes 27 us, not 16.
+__host__ __device__ inline int gemm_run(int units, int mper) {  // tiles of an XCD in a block of mper along M
+  return (units >> 3) * mper + (((units & 7) * mper + 7) >> 3);
+}
 inline unsigned gemm_grid(const GemmArgs& a) {
-  return 8u * (unsigned)((a.nblk * a.splits + 7) / 8) * (unsigned)a.mblk;
+  const int u = a.nblk * a.splits;
+  return 8u * (unsigned)(a.mblk / a.mper * gemm_run(u, a.mper) + gemm_run(u, a.mblk % a.mper));
 }
 __device__ __forceinline__ bool gemm_tile(const GemmArgs& a, int& u, int& mb) {
-  const int units = (a.nblk * a.splits + 7) >> 3;  // weight blocks x K parts of an XCD
-  const int j = (int)(blockIdx.x >> 3), blk = j / (units * a.mper), jj = j - blk * units * a.mper;
-  const int mper = min(a.mper, a.mblk - blk * a.mper);
-  u = (jj / mper) * 8 + (int)(blockIdx.x & 7);
-  mb = blk * a.mper + jj % mper;
-  return u < a.nblk * a.splits;
+  const int units = a.nblk * a.splits, run = gemm_run(units, a.mper), xcd = (int)(blockIdx.x & 7);
+  const int j = (int)(blockIdx.x >> 3), blk = j / run, jj = j - blk * run;
+  const int mper = min(a.mper, a.mblk - blk * a.mper), whole = (units >> 3) * mper;
+  if (jj < whole) {
+    u = (jj / mper) * 8 + xcd;
+    mb = blk * a.mper + jj % mper;
+    return true;
+  }
+  const int share = ((units & 7) * mper + 7) >> 3, i = xcd * share + jj - whole;
+  u = (units & ~7) + i / mper;
+  mb = blk * a.mper + i % mper;
+  return jj - whole < share && u < units;
 }
 
 // Epi(n, m, v, split): v[i] = the (partial) sum of weight row n + i and activation row m; n is a

@@ -44,14 +44,18 @@ __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ p, 
 
 // How a call of m rows runs. Tiles of 128 rows x 256 weight rows (k_gemm_big, one workgroup per CU) where
 // they nearly fill the 256 CUs: 512 / 2048 rows x 16384 x 2560 took 56 / 195 us, 64 x 64 tiles 75 / 290.
-// Else 64 x 64 tiles:
-// - up to 64 rows: four ways, and K cut until there are about 192 workgroups of at least four
-//   128-groups: 64 x 16384 x 2560 took 18 us with one way and 15 with four, 64 x 2560 x 8192 (40 tiles)
-//   36 us uncut and 12 in four parts;
-// - K cut until there are about 768 workgroups: 336 x 2576 x 2560 (246 tiles) took 24 us uncut, 17 in
-//   2 parts and 15 in 4; but from 320 tiles and for few groups two ways instead, as the launch that
-//   adds the parts costs 3-4 us: 512 x 2560 x 2560 (320 tiles) took 25 us with one way uncut, 20 in
-//   2 parts and 20 with two ways uncut, 512 x 3584 x 2560 (448 tiles) 25, 23 and 21.
+// Else 64 x 64 tiles; a CU holds one workgroup of four ways, two of two, three of one (us, weights from HBM):
+// - up to 256 tiles four ways (two where a part has fewer than 8 groups), and K cut while all parts' tiles still run at
+//   once: 333 x 2570 x 2560 (246 tiles) 25 with one way, 17 with two, 16 with four, 20 with one way in 2
+//   parts, whose sums cost a launch; 100 x 3584 x 2560 (112) 15 uncut, 13 in 2 parts; 64 x 2560 x 8192
+//   (40) 36 uncut with one way, 12 in 4 parts;
+// - beyond 32 groups, where those leave CUs idle (129 to 200 tiles) or there are more tiles: parts of one
+//   way for about 1536 workgroups: 200 x 2560 x 8192 (160 tiles) 34 in 4 parts, 38 with four ways; 333 x 2900
+//   x 8192 (276) 52 in 4 parts, 57 in 2, 66 with two ways; 600 x 3584 x 8192 (560) 93 in 2, 100 uncut; of
+//   12 groups at least: 97 x 12260 x 4224 (384, 33 groups) 43 in 4 parts, 40 in 2;
+// - else two ways, one beyond 512 tiles of at most 16 groups: 333 x 2900 x 2560 (276) 26 with one way, 23 with
+//   two, 24 in parts; 100 x 16384 x 2560 (512) 31 and 26, 2048 x 2560 x 2560 (1280) 58 and 56;
+//   389 x 11621 x 640 (1274) 22 and 24, 1355 x 10528 x 1024 (3630) 49 and 66.
 struct Plan {
   bool big;
   int ways, splits, gps;
@@ -62,18 +66,13 @@ Plan plan_rows(int m, int n, int k) {
   if ((int64_t)((m + 127) / 128) * ((n + 255) / 256) >= 224) return p;
   p.big = false;
   const int64_t tiles = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
-  int64_t s = 768 / tiles, most = 8;
-  if (m <= 64) {
-    p.ways = 4;
-    s = 192 / tiles;
-    most = 4;
-  } else if (tiles >= 320 && G <= 32) {
-    p.ways = 2;
-    s = 1;
-  }
-  const int parts = (int)std::max<int64_t>(1, std::min({most, s, (int64_t)G / 4}));
+  const bool few = tiles <= 256 && (G <= 32 || tiles <= 128 || tiles > 200);
+  const int64_t s = few ? 256 / tiles : G > 32 ? 1536 / tiles : 1;
+  const int parts = (int)std::max<int64_t>(1, std::min<int64_t>({4, s, G / (few ? 4 : 12)}));
   p.gps = (G + parts - 1) / parts;
   p.splits = (G + p.gps - 1) / p.gps;
+  if (few) p.ways = p.gps >= 8 ? 4 : 2;
+  else if (G <= 32 && (tiles <= 512 || G > 16)) p.ways = 2;
   return p;
 }
 

@@ -5,8 +5,7 @@ One "step" = one decoded token = ONE persistent cooperative kernel launch (fl_de
 the 40-layer 3B-class synthetic int4 model: all layers, final norm, tied bf16 LM head, greedy
 argmax. Tokens chain on the device (step i reads the token step i-1 wrote), so the timed loop
 has no host synchronisation. Weights are seeded random (no checkpoint exists); the prompt is
-512 seeded-uniform token ids prefilled before timing (through the verify kernel, 16 tokens per
-launch). After the timed decode, the speculative-verify latency (k = 4, 7 draft tokens at
+512 seeded-uniform token ids prefilled before timing (GEMM passes over up to 1024 tokens). After the timed decode, the speculative-verify latency (k = 4, 7 draft tokens at
 context 1024) is measured beside the decode latency at the same context.
 
 Prints ONE JSON line (the driver's contract) with `roofline` (HBM-bound: algorithmic bytes per
@@ -610,7 +609,7 @@ def main():
     prompt = torch.randint(0, args.vocab_size, (a.ctx,), generator=g, dtype=torch.int32).to(dev)
     seq = torch.empty(a.ctx + a.warmup + a.steps, dtype=torch.int32, device=dev)
     seq[:a.ctx] = prompt
-    log(f"prefill {a.ctx} tokens (verify kernel, 32 tokens per launch)")
+    log(f"prefill {a.ctx} tokens (GEMM passes over up to 1024 tokens)")
     from flint_amd.generate import prefill
     t0 = time.perf_counter()
     prefill(model, seq[:a.ctx - 1], 0)

@@ -155,7 +155,8 @@ class Engine {
   std::vector<torch::Tensor> keep_;
 };
 
-// WeightOnlyInt4Linear.forward (reference engine/quantize.py:517-525): y = x . dq^T, M <= 32 rows
+// WeightOnlyInt4Linear.forward (reference engine/quantize.py:517-525): y = x . dq^T, M <= 32 rows (the reference's
+// op form over torch tensors; more rows raise)
 torch::Tensor int4_linear(torch::Tensor x, torch::Tensor q, torch::Tensor sz, int64_t stream) {
   check_dev(x, torch::kBFloat16, "x");
   check_dev(q, torch::kInt32, "weight");

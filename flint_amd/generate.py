@@ -4,7 +4,7 @@ Mirrors reference engine/generate.py:57-81,137-206 (prefill / decode_one_token /
 generate) for greedy sampling and chat.py:71-96 (logits_at / pick / respond). Tokens stay on
 the device between steps: step i reads the token step i-1 wrote, so the loop issues launches
 back-to-back with no host synchronisation (gpt-fast's decode loop has none either). The prompt
-is prefilled through the speculative-verify kernel, up to 32 tokens per launch.
+runs as GEMM passes over up to 1024 tokens (fl_prefill), a short one through the verify kernel.
 """
 import torch
 

@@ -192,10 +192,12 @@ def test_weight_only_int4_linear(dev, lead):
 
 @pytest.mark.parametrize("m,n,k", [(33, 64, 128), (64, 63, 384), (65, 2570, 2560), (127, 130, 8192), (129, 16385, 256),
                                    (300, 16384, 128), (2049, 2048, 384), (8193, 65, 128), (400, 16385, 128),
-                                   (1100, 8200, 384), (2049, 4100, 256)])
+                                   (1100, 8200, 384), (2049, 4100, 256), (333, 2570, 1408), (130, 3400, 4352),
+                                   (300, 3500, 2304)])
 def test_gemm_rows(dev, m, n, k):
     """fl_gemm_rows_int4 at the edges of its tiles (64 and 128 rows of both operands, and 128 x 256 where
-    at least 224 of those fill the chip: the last three), of its K parts and of its launches of 8192 rows, N odd and not, into an output that is not 8-byte aligned
+    at least 224 of those fill the chip: m = 400, 1100 and 2049 with n = 4100), of its ways, its K parts
+    and its launches of 8192 rows, N odd and not, into an output that is not 8-byte aligned
     too: fp32 sums of exact products, so a result may differ from the oracle's only where another
     order of the sum rounds to the neighbouring bf16 value."""
     from flint_amd.quantize import dequantize_int4, gemm_int4, quantize_int4

@@ -110,17 +110,23 @@ int fl_gemm_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint1
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const GemmArgs a{q, sz, x, m, n, k, 0, 0, 1, k / FL_GROUP, 0};
   const EpiBf16 epi = out_bf16(y, m, n);
-  // One workgroup per 64 weight rows (four ways) where that gives at least 192, else one per 16 rows
-  // with as many ways as the LDS holds: 32 rows x 16384 x 2560 12 us (four ways; 23 in the former
-  // kernel, which re-read X from L2 per 16 weight rows), 5 rows x 2560 x 8192 9.7 us (sixteen ways;
-  // 12.2, four waves whose 16 loads each waited for the one before), 32 rows 13.7 us (eight ways).
-  const bool wide = (n + 63) / 64 >= 192;
+  // As many ways as fit while all workgroups run at once, in 16-row tiles up to one per CU, else 32-row
+  // ones, else fewer ways (us, weights from HBM; the former four-wave kernel, which re-read X per
+  // tile and waited for each of its loads, in brackets): 5 rows x 2560 x 8192 (160 tiles of 16) sixteen ways 11,
+  // eight 12 (23); 12 rows x 6000 x 5120 (375) sixteen ways 17, eight over 32 rows 12 (18); 12 rows x 10477 x 3456 (655)
+  // sixteen 18, eight 14, four 12 (15); 12 rows x 16384 x 2560 (1024) four over 32 rows 11.7, over 16 or 64 12 (15).
+  // 17 to 32 rows hold twice the X: 2560 x 8192 eight ways 15 (29); 6000 x 5120 eight over 16 rows 19, over 32 rows 14
+  // (25); 12000 x 8192 (750) eight 41 and 37, four over 32 rows 33 (53); 16384 x 2560 24, 16, 13 (22).
+  const int t16 = (n + 15) / 16;
   if (m <= 16) {
-    if (wide) launch<4, 4, 1, 1>(a, epi, s);
-    else launch<1, 16, 1, 1>(a, epi, s);
+    if (t16 <= 256) launch<1, 16, 1, 1>(a, epi, s);
+    else if (t16 <= 512) launch<2, 8, 1, 1>(a, epi, s);
+    else if (t16 <= 896) launch<1, 4, 1, 1>(a, epi, s);
+    else launch<2, 4, 1, 1>(a, epi, s);
   } else {
-    if (wide) launch<4, 4, 1, 2>(a, epi, s);
-    else launch<1, 8, 1, 2>(a, epi, s);
+    if (t16 <= 256) launch<1, 8, 1, 2>(a, epi, s);
+    else if (t16 <= 512) launch<2, 8, 1, 2>(a, epi, s);
+    else launch<2, 4, 1, 2>(a, epi, s);
   }
   return hipGetLastError() == hipSuccess ? FL_OK : FL_E_LAUNCH;
 }

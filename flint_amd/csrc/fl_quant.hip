@@ -30,7 +30,8 @@ __global__ __launch_bounds__(256) void k_quantize(const uint16_t* __restrict__ w
     v[0] = reinterpret_cast<const uint4*>(w)[word];
     v[1] = reinterpret_cast<const uint4*>(w)[word + 8];
   }
-  float x[2][8], mx = -INFINITY, mn = INFINITY;
+  // from the first element on: fmaxf / fminf drop a NaN, so that only a group of NaN alone gives NaN
+  float x[2][8], mx = bflo(v[0].x), mn = mx;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const uint32_t pk[4] = {v[i].x, v[i].y, v[i].z, v[i].w};

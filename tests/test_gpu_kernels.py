@@ -338,6 +338,38 @@ def test_quantize_wide_range(dev, kind):
     assert bool(fine.all()) == (kind != "inf")
 
 
+def test_quantize_nan(dev):
+    """A group of only NaN has a NaN zero point (torch's min of it) and the scale of an empty range; in a
+    group with other values NaN takes no part in the range and becomes 0. The other groups of the wave
+    are what they are without it."""
+    from flint_amd.quantize import quantize_int4, unpack_q, unpack_sz
+    n, k = 37, 384
+    w = _weights(n, k, 32).to(dev)
+    base_q, base_sz = quantize_int4(w)
+    bad = w.clone()
+    bad[3, :128] = float("nan")
+    bad[::5, 256:384] = float("nan")
+    some = torch.zeros(n, k, dtype=torch.bool, device=dev)
+    some[7, 0], some[8, 131], some[9, 128:255] = True, True, True
+    bad[some] = float("nan")
+    q, sz = quantize_int4(bad)
+    gone = torch.isnan(bad.view(n, -1, 128)).all(2)
+    s, z = unpack_sz(sz)
+    v = unpack_q(q).view(n, -1, 128)
+    assert bool(torch.isnan(z[gone]).all()) and not bool(v[gone].any())
+    tiny = torch.tensor(1e-6, dtype=torch.bfloat16, device=dev) / 15
+    assert bool((s[gone] == tiny).all())
+    part = some.view(n, -1, 128).any(2)
+    clean = ~gone & ~part
+    assert torch.equal(v[clean], unpack_q(base_q).view(n, -1, 128)[clean])
+    assert torch.equal(sz[clean], base_sz[clean])
+    fill = torch.where(some, bad.view(n, -1, 128).nan_to_num(-1e9).amax(2).repeat_interleave(128, 1), w)
+    fq, fsz = quantize_int4(fill.to(torch.bfloat16))
+    assert torch.equal(sz[part], fsz[part]) and not bool(unpack_q(q)[some].any())
+    keep = part.repeat_interleave(128, 1) & ~some
+    assert torch.equal(unpack_q(q)[keep], unpack_q(fq)[keep])
+
+
 @pytest.mark.parametrize("n,k", [(16, 128), (32, 256), (48, 640), (16, 16384), (160, 1152)])
 def test_tile_layout(dev, n, k):
     """fl_tile_int4 at group counts that do and do not fill its workgroups of four, against the layout

@@ -88,6 +88,72 @@ void launch_small(int ways, const GemmArgs& a, Epi epi, hipStream_t s) {
   else launch<4, 1, 1, 4>(a, epi, s);
 }
 
+// The former kernel of 2 to 32 rows, kept for few K groups: one workgroup of four waves per 16 weight rows,
+// the groups round-robin over the waves, X fragments straight from global memory (rows past M or N read as zeros),
+// one barrier for the waves' sums, added in wave order. It starts up faster (3.5 us where k_gemm_rows takes 4.9: 8 x 2560
+// x 512), but waits for each group's loads in turn and reads X once per 16 weight rows.
+constexpr int kGemmWaves = 4;
+
+__global__ __launch_bounds__(64 * kGemmWaves) void k_gemm(const uint32_t* __restrict__ q,
+                                                          const uint32_t* __restrict__ sz,
+                                                          const uint16_t* __restrict__ x,
+                                                          uint16_t* __restrict__ y, int m, int n,
+                                                          int k) {
+  __shared__ float part[kGemmWaves][2][256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, c = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  const int rows = min(16, n - n0);
+  const int groups = k >> 7;
+  const bool two = m > 16;  // a second 16-row block of activations (tokens 16..31)
+  const auto wr = buf_rsrc(q + (size_t)n0 * (k >> 3), (uint32_t)rows * (uint32_t)(k >> 1));
+  const auto sr = buf_rsrc(sz + (size_t)n0 * groups, (uint32_t)rows * (uint32_t)groups * 4u);
+  const auto xr = buf_rsrc(x, (uint32_t)m * (uint32_t)k * 2u);
+  const uint32_t woff = (uint32_t)r * (uint32_t)(k >> 1) + (uint32_t)c * 16u;   // bytes
+  const uint32_t xoff = (uint32_t)r * (uint32_t)k * 2u + (uint32_t)c * 64u;     // bytes
+  const uint32_t xoff2 = xoff + 16u * (uint32_t)k * 2u;
+  fl_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, acc2 = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int u = wave; u < groups; u += kGemmWaves) {
+    const uint4 w = buf_ld128(wr, woff + (uint32_t)u * 64u);
+    const uint32_t s = buf_ld32(sr, ((uint32_t)r * (uint32_t)groups + (uint32_t)u) * 4u);
+    uint4 xa[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) xa[e] = buf_ld128(xr, xoff + (uint32_t)u * 256u + (uint32_t)e * 16u);
+    uint32_t d[4][4];
+    dq32(w, dq_const(s), d);
+    mfma_chunk(d, xa, acc);
+    if (two) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) xa[e] = buf_ld128(xr, xoff2 + (uint32_t)u * 256u + (uint32_t)e * 16u);
+      mfma_chunk(d, xa, acc2);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    part[wave][0][(c * 4 + i) * 16 + r] = acc[i];
+    part[wave][1][(c * 4 + i) * 16 + r] = acc2[i];
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < (two ? 512 : 256); t += 64 * kGemmWaves) {
+    const int row = t >> 4, col = t & 15;  // activation row (token), weight row in the tile
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kGemmWaves; ++w) v += part[w][t >> 8][t & 255];
+    if (row < m && col < rows) y[(size_t)row * n + n0 + col] = (uint16_t)f2bf(v);
+  }
+}
+
+// k_gemm against k_gemm_rows at m rows, t16 blocks of 16 weight rows and G groups (us, weights from HBM, k_gemm
+// first): up to 16 rows 2 x 2560 x 1024 5.0 / 5.5, x 1280 5.7 / 5.6, x 1536 6.3 / 5.7; beyond 768 blocks, where
+// k_gemm_rows has fewer ways, 2 x 16384 x 2048 11.2 / 11.5, x 2560 13.3 / 13.3, x 3072 15.1 / 14.6; with more rows
+// earlier, by the products in all: 16 x 16384 x 768 7.2 / 7.7, x 1024 9.0 / 8.3. More than 16 rows read X twice per
+// weight: 17 x 2560 x 768 5.0 / 5.1, x 1024 5.4 / 5.4; 32 x 8192 x 512 5.5 / 5.8, 32 x 12288 x 512 6.8 / 6.2; one or
+// two groups always: 32 x 49152 x 128 8.3 / 11.2.
+bool few_groups(int m, int t16, int G) {
+  const int64_t work = (int64_t)m * t16 * G;
+  return m <= 16 ? G <= (t16 <= 768 ? 10 : 20) && (G == 1 || work < 131072) : G <= 2 || (G <= 6 && work <= 65536);
+}
+
 EpiBf16 out_bf16(uint16_t* y, int m, int n) {
   return EpiBf16{y, m, n, n % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0};
 }
@@ -118,7 +184,9 @@ int fl_gemm_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint1
   // 17 to 32 rows hold twice the X: 2560 x 8192 eight ways 15 (29); 6000 x 5120 eight over 16 rows 19, over 32 rows 14
   // (25); 12000 x 8192 (750) eight 41 and 37, four over 32 rows 33 (53); 16384 x 2560 24, 16, 13 (22).
   const int t16 = (n + 15) / 16;
-  if (m <= 16) {
+  if (few_groups(m, t16, k / FL_GROUP)) {
+    hipLaunchKernelGGL(k_gemm, dim3(t16), dim3(64 * kGemmWaves), 0, s, q, sz, x, y, m, n, k);
+  } else if (m <= 16) {
     if (t16 <= 256) launch<1, 16, 1, 1>(a, epi, s);
     else if (t16 <= 512) launch<2, 8, 1, 1>(a, epi, s);
     else if (t16 <= 896) launch<1, 4, 1, 1>(a, epi, s);

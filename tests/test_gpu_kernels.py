@@ -190,6 +190,18 @@ def test_weight_only_int4_linear(dev, lead):
         mod(torch.zeros(4, k + 128, dtype=torch.bfloat16, device=dev))  # wrong inner dimension
 
 
+def _check_gemm(y, x, dq):
+    """y = bf16 of an fp32 sum of the exact products x . dq^T, in any order of steps of 32 products: at most
+    32 roundings within a step's own products, one per step of the accumulator, 16 where parts meet, each
+    of 2^-23 of the magnitudes that it adds; then half a bf16 ulp."""
+    xd, dd = x.double(), dq.double()
+    ref = xd @ dd.T
+    bound = (x.shape[1] / 32 + 48) * 2.0 ** -23 * (xd.abs() @ dd.abs().T) + ref.abs() * 2.0 ** -8
+    d = (y.double() - ref).abs()
+    log(f"gemm {tuple(x.shape)} -> {y.shape[1]}: max|d| {float(d.max()):.3e}, largest share of its bound {float((d / bound).max()):.3f}")
+    assert bool((d <= bound).all())
+
+
 @pytest.mark.parametrize("m,n,k", [(33, 64, 128), (64, 63, 384), (65, 2570, 2560), (127, 130, 8192), (129, 16385, 256),
                                    (300, 16384, 128), (2049, 2048, 384), (8193, 65, 128), (400, 16385, 128),
                                    (1100, 8200, 384), (2049, 4100, 256), (333, 2570, 1408), (130, 3400, 4352),
@@ -215,6 +227,19 @@ def test_gemm_rows(dev, m, n, k):
     buf = torch.zeros(m * n + 3, dtype=torch.bfloat16, device=dev)
     gemm_int4(q, sz, x, buf[1:1 + m * n].view(m, n))
     assert torch.equal(buf[1:1 + m * n].view(m, n), y) and not buf[:1].any() and not buf[1 + m * n:].any()
+
+
+@pytest.mark.parametrize("m,n,k", [(2, 5, 128), (16, 131073, 128), (9, 2561, 1280), (9, 2561, 1408), (3, 12305, 2560),
+                                   (3, 12305, 2688), (16, 13000, 1280), (16, 13109, 1280), (17, 2561, 768), (17, 2561, 896),
+                                   (32, 5440, 768), (32, 5500, 768), (25, 20003, 256), (17, 16384, 384)])
+def test_gemm_few_groups(dev, m, n, k):
+    """fl_gemm_int4 on both sides of each line between its two kernels (few K groups: k_gemm): 10 and 20
+    groups, 131072 products (by 16 rows and 128 columns) up to 16 rows; 2 and 6 groups, 65536 beyond."""
+    from flint_amd.quantize import dequantize_int4, gemm_int4, quantize_int4
+    w = _weights(n, k, 23, "edge").to(dev)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(24)).to(torch.bfloat16).to(dev)
+    q, sz = quantize_int4(w)
+    _check_gemm(gemm_int4(q, sz, x), x, dequantize_int4(q, sz))
 
 
 def test_scales_and_zeros_gptfast_layout(dev):

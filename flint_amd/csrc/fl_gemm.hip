@@ -176,20 +176,21 @@ int fl_gemm_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint1
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const GemmArgs a{q, sz, x, m, n, k, 0, 0, 1, k / FL_GROUP, 0};
   const EpiBf16 epi = out_bf16(y, m, n);
-  // As many ways as fit while all workgroups run at once, in 16-row tiles up to one per CU, else 32-row
-  // ones, else fewer ways (us, weights from HBM; the former four-wave kernel, which re-read X per
-  // tile and waited for each of its loads, in brackets): 5 rows x 2560 x 8192 (160 tiles of 16) sixteen ways 11,
-  // eight 12 (23); 12 rows x 6000 x 5120 (375) sixteen ways 17, eight over 32 rows 12 (18); 12 rows x 10477 x 3456 (655)
-  // sixteen 18, eight 14, four 12 (15); 12 rows x 16384 x 2560 (1024) four over 32 rows 11.7, over 16 or 64 12 (15).
-  // 17 to 32 rows hold twice the X: 2560 x 8192 eight ways 15 (29); 6000 x 5120 eight over 16 rows 19, over 32 rows 14
-  // (25); 12000 x 8192 (750) eight 41 and 37, four over 32 rows 33 (53); 16384 x 2560 24, 16, 13 (22).
+  // k_gemm_rows, up to 16 rows: sixteen ways over 16 weight rows while one workgroup per CU holds them all (256
+  // blocks of 16), eight over 32 up to two blocks per CU, then four: over 16 weight rows while that gives a CU
+  // three blocks where 32 would give it four (8 rows x 11200 x 5120, 700 blocks, 22.6 us and 24.5), over 32 beyond
+  // (12800, 800 blocks, 26.5 and 25.0; X is read half as often). 5 x 2560 x 8192 sixteen ways 11, eight 12; 12 x 6000 x
+  // 5120 (375) sixteen 17, eight over 32 rows 12; 12 x 10477 x 3456 (655) sixteen 18, eight 14, four 12.
+  // 17 to 32 rows hold twice the X in LDS, so eight ways at most: 32 x 2560 x 8192 15; 6000 x 5120 (375) eight over 16
+  // weight rows 19, over 32 14; beyond 512 blocks four over 32: 12000 x 8192 (750) eight 37 to 41, four 33; 16384 x
+  // 2560 eight over 16 rows 24, over 32 16, four 13.
   const int t16 = (n + 15) / 16;
   if (few_groups(m, t16, k / FL_GROUP)) {
     hipLaunchKernelGGL(k_gemm, dim3(t16), dim3(64 * kGemmWaves), 0, s, q, sz, x, y, m, n, k);
   } else if (m <= 16) {
     if (t16 <= 256) launch<1, 16, 1, 1>(a, epi, s);
     else if (t16 <= 512) launch<2, 8, 1, 1>(a, epi, s);
-    else if (t16 <= 896) launch<1, 4, 1, 1>(a, epi, s);
+    else if (t16 <= 768) launch<1, 4, 1, 1>(a, epi, s);
     else launch<2, 4, 1, 1>(a, epi, s);
   } else {
     if (t16 <= 256) launch<1, 8, 1, 2>(a, epi, s);

@@ -180,8 +180,8 @@ torch::Tensor int4_linear(torch::Tensor x, torch::Tensor q, torch::Tensor sz, in
 }
 
 // The module's forward in one call, for the arguments it can take as they are; None for any other
-// (another dtype or device, strides, a wrong inner dimension): the caller's general path decides
-// those. One row runs the GEMV, up to 32 the GEMM, more the GEMM over rows with a workspace of
+// (another dtype or device, strides, a wrong inner dimension) and where memory runs out: the caller's
+// general path decides those. One row runs the GEMV, up to 32 the GEMM, more the GEMM over rows with a workspace of
 // torch's. From Python the same steps (checks, allocation, ctypes) cost 14 us a call, more than
 // the kernels of one token; here about 5.
 pybind11::object linear_fast(const torch::Tensor& x, const torch::Tensor& q, const torch::Tensor& sz, int64_t stream) {
@@ -198,8 +198,8 @@ pybind11::object linear_fast(const torch::Tensor& x, const torch::Tensor& q, con
   if (m > FL_MAX_VERIFY && fl_gemm_rows_workspace((int32_t)m, (int32_t)n, (int32_t)k, &ws_bytes) != FL_OK)
     return pybind11::none();
   torch::Tensor y;
-  int rc;
-  {
+  int rc = FL_E_HIP;
+  try {
     pybind11::gil_scoped_release nogil;  // a launch may wait for room in the queue
     auto sizes = x.sizes().vec();
     sizes.back() = n;
@@ -218,8 +218,9 @@ pybind11::object linear_fast(const torch::Tensor& x, const torch::Tensor& q, con
       rc = fl_gemm_rows_int4(qp, sp, xp, yp, ws_bytes > 0 ? ws.data_ptr<float>() : nullptr, (int32_t)m, (int32_t)n,
                              (int32_t)k, stream_of(stream));
     }
+  } catch (const c10::OutOfMemoryError&) {
   }
-  if (rc != FL_OK) return pybind11::none();  // the general path raises it
+  if (rc != FL_OK) return pybind11::none();  // the general path raises it, or runs without the workspace
   return pybind11::cast(y);
 }
 

@@ -93,7 +93,8 @@ def gemv_int4(q, sz, x, y=None):
 def gemm_int4(q, sz, x, y=None):
     """Y[M,N] = bf16(X[M,K] . dq[N,K]^T) for any M: one fl_gemm_int4 launch up to 32 rows
     (FL_MAX_VERIFY), which reads the weights once for all of them; beyond, fl_gemm_rows_int4, which
-    reads and dequantises them once per 64 or 128 rows."""
+    reads and dequantises them once per 64 or 128 rows (launches of 32 rows where it does not take the
+    size or there is no memory for its workspace)."""
     _check_dev(q, torch.int32, "q")
     _check_dev(sz, torch.int32, "sz")
     _check_dev(x, torch.bfloat16, "x")
@@ -108,10 +109,14 @@ def gemm_int4(q, sz, x, y=None):
     if m > _lib.MAX_VERIFY:
         need = _lib.ctypes.c_int64()
         if _lib.load().fl_gemm_rows_workspace(m, n, k, _lib.ctypes.byref(need)) == _lib.FL_OK:
-            ws = torch.empty(need.value // 4, dtype=torch.float32, device=q.device) if need.value else None
-            _lib.call("fl_gemm_rows_int4", _lib.ptr(q), _lib.ptr(sz), _lib.ptr(x), _lib.ptr(y), _lib.ptr(ws),
-                      m, n, k, _lib.stream_ptr())
-            return y
+            try:
+                ws = torch.empty(need.value // 4, dtype=torch.float32, device=q.device) if need.value else None
+            except torch.OutOfMemoryError:
+                pass  # no room for the part sums: launches of 32 rows need none
+            else:
+                _lib.call("fl_gemm_rows_int4", _lib.ptr(q), _lib.ptr(sz), _lib.ptr(x), _lib.ptr(y), _lib.ptr(ws),
+                          m, n, k, _lib.stream_ptr())
+                return y
     for r0 in range(0, m, _lib.MAX_VERIFY):
         mb = min(_lib.MAX_VERIFY, m - r0)
         _lib.call("fl_gemm_int4", _lib.ptr(q), _lib.ptr(sz), _lib.ptr(x[r0:]), _lib.ptr(y[r0:]), mb, n, k,

@@ -449,3 +449,31 @@ def test_linear_module_call(dev, shape):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, mod(x * (i + 1)))
+
+
+def test_linear_without_workspace(dev):
+    """Where memory has no room for the part sums of more than 32 rows, the call runs in launches of 32
+    rows instead, through the module's single-call forward and through gemm_int4."""
+    from flint_amd import _lib
+    from flint_amd import quantize as Q
+    m, n, k = 100, 2560, 8192  # 4 MB of part sums, a result of 512 KB
+    need = _lib.ctypes.c_int64()
+    _lib.call("fl_gemm_rows_workspace", m, n, k, _lib.ctypes.byref(need))
+    assert need.value > 2 << 20
+    mod = Q.WeightOnlyInt4Linear.from_float(_weights(n, k, 51).to(dev))
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(52)).to(torch.bfloat16).to(dev)
+    want = torch.cat([Q.gemm_int4(mod.weight, mod.scales_and_zeros, x[r:r + 32].contiguous()) for r in range(0, m, 32)])
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    # room for the result in segments of the allocator that stay; no new segments, the larger ones filled up
+    parts = [torch.empty(900 << 10, dtype=torch.uint8, device=dev) for _ in range(8)]
+    del parts[::2]
+    torch.cuda.set_per_process_memory_fraction(0.0)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            for _ in range(1000):
+                parts.append(torch.empty(2 << 20, dtype=torch.uint8, device=dev))
+        got, got2 = mod(x), Q.gemm_int4(mod.weight, mod.scales_and_zeros, x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got, want) and torch.equal(got2, want)

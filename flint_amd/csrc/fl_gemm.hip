@@ -43,7 +43,10 @@ __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ p, 
 }
 
 // How a call of m rows runs. Tiles of 128 rows x 256 weight rows (k_gemm_big, one workgroup per CU) where
-// they nearly fill the 256 CUs: 512 / 2048 rows x 16384 x 2560 took 56 / 195 us, 64 x 64 tiles 75 / 290.
+// they nearly fill the 256 CUs: 512 / 2048 rows x 16384 x 2560 56 / 201 us, 64 x 64 tiles 89 / 340. A second round that
+// is half empty still costs a whole one, which up to 12 groups is more than the smaller tiles take: 576 rows x
+// 16384 (320 tiles) x 640 35 and 31, x 1280 54 and 52, x 2560 92 and 97; 700 x 12288 (288) x 1280 54 and 49; 768 x 16384
+// (384) x 640 37 and 38; one or two groups do not pay for the large tiles' start-up: 448 x 12288 x 256 15 and 14.
 // Else 64 x 64 tiles; a CU holds one workgroup of four ways, two of two, three of one (us, weights from HBM):
 // - up to 256 tiles four ways (two where a part has fewer than 8 groups), and K cut while all parts' tiles still run at
 //   once: 333 x 2570 x 2560 (246 tiles) 25 with one way, 17 with two, 16 with four, 20 with one way in 2
@@ -63,7 +66,8 @@ struct Plan {
 Plan plan_rows(int m, int n, int k) {
   const int G = k / FL_GROUP;
   Plan p{true, 1, 1, G};
-  if ((int64_t)((m + 127) / 128) * ((n + 255) / 256) >= 224) return p;
+  const int64_t big = (int64_t)((m + 127) / 128) * ((n + 255) / 256);
+  if (big >= 224 && G > 2 && (big <= 256 || big >= 384 || G > 12)) return p;
   p.big = false;
   const int64_t tiles = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
   const bool few = tiles <= 256 && (G <= 32 || tiles <= 128 || tiles > 200);

@@ -461,7 +461,9 @@ void pf_launch(GemmArgs a, Epi epi, hipStream_t s) {
 // returns their number. Measured at flint-3b's sizes (us, weights from HBM):
 // - tiles of 256 x 128 (k_gemm_big, one workgroup per CU) where they and the parts give at least 160
 //   workgroups: gate/up at 512 / 1024 tokens (256 / 512 tiles) 53 / 101, 57 / 115 in tiles of 128 x 128; down at
-//   512 (40 tiles) 39 in four parts, 42 in tiles of 64 x 64; O at 512 has too few groups for four parts of eight;
+//   512 (40 tiles) 39 in four parts, 42 in tiles of 64 x 64; O at 512 has too few groups for four parts of eight; not
+//   where a second round would be half empty or more: gate/up at 576 / 768 tokens (320 / 384) cost 12 / 8 us a layer more
+//   than in tiles of 128 x 128, at 896 (448) 8 less;
 // - else tiles of 64 x 64, up to 256 of them four ways, up to 512 two: QKV at 64 / 512 tokens (56 / 448 tiles)
 //   20 / 27 with one way, 14 / - with four, - / 24 with two; gate/up at 64 (256) 21 and 15; parts of about ten
 //   groups, four at most, more while they give fewer than 160 workgroups: O at 512 (320 tiles) 19 in two parts,
@@ -480,7 +482,8 @@ int pf_gemm(const uint32_t* qt, const uint32_t* sz, const uint16_t* x, int T, in
     a.splits = (G + a.gps - 1) / a.gps;
   };
   if (parts) cut(256 / t256, 8);
-  if (t256 * a.splits >= 160) {
+  const int big = t256 * a.splits;
+  if (big >= 160 && (big <= 256 || big > 384)) {
     a.tile(256, 128);
     hipLaunchKernelGGL((k_gemm_big<true, 8, 4, Epi>), dim3(gemm_grid(a)), dim3(512), 0, s, a, epi);
     return a.splits;

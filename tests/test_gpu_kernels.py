@@ -206,10 +206,11 @@ def _check_gemm(y, x, dq):
                                    (300, 16384, 128), (2049, 2048, 384), (8193, 65, 128), (400, 16385, 128),
                                    (1100, 8200, 384), (2049, 4100, 256), (333, 2570, 1408), (130, 3400, 4352),
                                    (300, 3500, 2304), (2, 4097, 384), (16, 8193, 128), (9, 14350, 640), (17, 4097, 1152),
-                                   (32, 8193, 640), (9, 12270, 2688), (16, 12300, 1536)])
+                                   (32, 8193, 640), (9, 12270, 2688), (16, 12300, 1536), (400, 14400, 384), (448, 14340, 256),
+                                   (520, 13000, 1536), (520, 13000, 1664), (1100, 10900, 384)])
 def test_gemm_rows(dev, m, n, k):
     """fl_gemm_rows_int4 at the edges of its tiles (64 and 128 rows of both operands, and 128 x 256 where
-    at least 224 of those fill the chip: m = 400, 1100 and 2049 with n = 4100), of its ways, its K parts
+    at least 224 of those fill the chip, beyond 256 from 384 or 13 groups on: 400 x 14400, 520 x 13000 x 1664, 1100 x 10900), of its ways, its K parts
     and its launches of 8192 rows, and fl_gemm_int4 past 256, 512 and 768 tiles of 16 weight rows, N odd and not, into an output that is not 8-byte aligned
     too: fp32 sums of exact products, so a result may differ from the oracle's only where another
     order of the sum rounds to the neighbouring bf16 value."""

@@ -48,11 +48,11 @@ def test_prefill_small(dev, n, pos):
 
 
 @pytest.mark.parametrize("name,n,pos", [("tiny", 1000, 0), ("tiny", 40, 900), ("tiny", 20, 1000), ("flint-3b-l1", 100, 2000),
-                                        ("wide", 90, 7), ("42 heads", 840, 2100)])
+                                        ("wide", 90, 7), ("42 heads", 840, 2100), ("flint-3b-l1", 600, 0)])
 def test_prefill_shapes(dev, name, n, pos):
     """Few KV heads; a short prompt behind many keys (key parts); the 3B layer; the widest rows; enough
     rows for the large GEMM tiles (2688 weight rows: the last tile is half empty) and, behind enough
-    keys, for the attention's one-way form."""
+    keys, for the attention's one-way form; 320 large tiles, where gate/up takes smaller ones."""
     over = {}
     if name == "42 heads":
         name, over = "flint-3b-l1", dict(n_head=42, n_local_heads=3, dim=2688, vocab_size=2048)

@@ -50,6 +50,15 @@ def ulp_stats(e, r):
             "top": float((d / top).max())}
 
 
+def gemm_bound(x, dq):
+    """(fp64 x . dq^T, the largest distance of bf16 of an fp32 sum of its exact products from it). The sum may
+    go in any order of steps of 32 products: at most 32 roundings within a step, one per step of the
+    accumulator and 16 where parts meet, each of 2^-23 of the magnitudes that it adds; then half a bf16 ulp."""
+    xd, dd = x.double(), dq.double()
+    ref = xd @ dd.T
+    return ref, (x.shape[1] / 32 + 48) * 2.0 ** -23 * (xd.abs() @ dd.abs().T) + ref.abs() * 2.0 ** -8
+
+
 def make_pair(name, seed=0, n_layer=None, device="cuda", weight_device="cpu", **over):
     """(args, sd, engine, oracle) for config `name` with identical bf16 master weights."""
     from flint_amd.model import Transformer

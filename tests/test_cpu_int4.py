@@ -18,7 +18,7 @@ from flint_amd.synth import CONFIGS, ModelArgs, synth_weights
 from oracle import quant
 from oracle.cpu_int4 import CpuInt4Decoder, CpuInt4Linear
 from oracle.model import OracleModel
-from tests.helpers import log, logit_stats, near_tie, top2_margin
+from tests.helpers import gemm_bound, log, logit_stats, near_tie, top2_margin
 
 CPU_BAR_MAX = 0.1875
 CPU_BAR_MEAN = 0.04
@@ -75,3 +75,20 @@ def test_cpu_int4_decoder_matches_oracle(name):
             f"argmax {int(ld.argmax())}/{int(lr.argmax())} margin {top2_margin(lr):.4f}")
         assert st["max"] <= CPU_BAR_MAX and st["mean"] <= CPU_BAR_MEAN
         assert int(ld.argmax()) == int(lr.argmax()) or near_tie(lr, CPU_BAR_MAX)
+
+
+def test_gemm_bound_catches_a_product():
+    """The bound that the GEMM kernels are tested with holds for an fp32 sum, and one product left out of each
+    sum, at the largest K tested, breaks it in many of the results."""
+    m, n, k = 16, 96, 8192
+    g = torch.Generator().manual_seed(61)
+    dq = quant.dq_linear_weight((torch.randn(n, k, generator=g) * 0.02).to(torch.bfloat16))
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    ref, bound = gemm_bound(x, dq)
+    y = x.float() @ dq.float().T
+    assert bool(((y.to(torch.bfloat16).double() - ref).abs() <= bound).all())
+    j = torch.randint(0, k, (m, n), generator=g)
+    slip = y - x.float().gather(1, j) * dq.float()[torch.arange(n), j]
+    share = float(((slip.to(torch.bfloat16).double() - ref).abs() > bound).float().mean())
+    log(f"one product left out: {share:.2f} of the results past the bound")
+    assert share > 0.25

@@ -6,7 +6,7 @@ fp32-accumulation bound of an fp64 brute force, rounded to bf16.
 import pytest
 import torch
 
-from tests.helpers import log
+from tests.helpers import gemm_bound, log
 
 pytestmark = pytest.mark.gpu
 
@@ -191,12 +191,7 @@ def test_weight_only_int4_linear(dev, lead):
 
 
 def _check_gemm(y, x, dq):
-    """y = bf16 of an fp32 sum of the exact products x . dq^T, in any order of steps of 32 products: at most
-    32 roundings within a step's own products, one per step of the accumulator, 16 where parts meet, each
-    of 2^-23 of the magnitudes that it adds; then half a bf16 ulp."""
-    xd, dd = x.double(), dq.double()
-    ref = xd @ dd.T
-    bound = (x.shape[1] / 32 + 48) * 2.0 ** -23 * (xd.abs() @ dd.abs().T) + ref.abs() * 2.0 ** -8
+    ref, bound = gemm_bound(x, dq)
     d = (y.double() - ref).abs()
     log(f"gemm {tuple(x.shape)} -> {y.shape[1]}: max|d| {float(d.max()):.3e}, largest share of its bound {float((d / bound).max()):.3f}")
     assert bool((d <= bound).all())
@@ -218,13 +213,8 @@ def test_gemm_rows(dev, m, n, k):
     w = _weights(n, k, 21, "edge").to(dev)
     x = torch.randn(m, k, generator=torch.Generator().manual_seed(22)).to(torch.bfloat16).to(dev)
     q, sz = quantize_int4(w)
-    ref = x.float() @ dequantize_int4(q, sz).float().T
-    # |fp32 sum - exact| <= K 2^-24 sum |x w|, and half a bf16 ulp of the result
-    bound = k * 2.0 ** -23 * (x.float().abs() @ dequantize_int4(q, sz).float().abs().T) + ref.abs() * 2.0 ** -8
     y = gemm_int4(q, sz, x)
-    d = (y.float() - ref).abs()
-    log(f"gemm rows {m} x {n} x {k}: max|d| {float(d.max()):.3e}, largest share of its bound {float((d / bound).max()):.3f}")
-    assert bool((d <= bound).all())
+    _check_gemm(y, x, dequantize_int4(q, sz))
     buf = torch.zeros(m * n + 3, dtype=torch.bfloat16, device=dev)
     gemm_int4(q, sz, x, buf[1:1 + m * n].view(m, n))
     assert torch.equal(buf[1:1 + m * n].view(m, n), y) and not buf[:1].any() and not buf[1 + m * n:].any()

@@ -9,13 +9,13 @@ from tests.helpers import check_rows, fill_kv_random, log, make_pair, oracle_pai
 pytestmark = pytest.mark.gpu
 
 
-def _check(name, eng, orc, n, pos, seed):
+def _check(name, eng, orc, n, pos, seed, chunk=32):
     from flint_amd.generate import prefill
     args = eng.config
     if pos:
         fill_kv_random(eng, orc, pos, seed=seed)
     toks = torch.randint(0, args.vocab_size, (n + 1,), generator=torch.Generator().manual_seed(seed), dtype=torch.int32)
-    nxt = prefill(eng, toks[:n].to(eng.device), pos)
+    nxt = prefill(eng, toks[:n].to(eng.device), pos, chunk=chunk)
     lg = torch.empty(args.vocab_size, dtype=torch.float32, device=eng.device)
     eng.decode_step(toks[n:].to(eng.device), pos + n, logits=lg)
     eng.check()
@@ -45,6 +45,24 @@ def test_prefill_small(dev, n, pos):
     eng.setup_caches(1, 1100)
     orc.setup_caches(eng.max_seq_length)
     _check("small", eng, orc, n, pos, seed=n)
+
+
+@pytest.mark.parametrize("chunk", [16, 31, "no memory"])
+def test_prefill_verify_launches(dev, chunk, monkeypatch):
+    """A prompt over several verify launches, the last one partial: with a chunk below 32, and with the default
+    one where memory has no room for fl_prefill's workspace."""
+    args, sd, eng, orc = make_pair("small", seed=3)
+    eng.setup_caches(1, 128)
+    orc.setup_caches(eng.max_seq_length)
+    asked = []
+
+    def refuse(*a):
+        asked.append(a)
+        raise torch.OutOfMemoryError("no room")
+
+    monkeypatch.setattr(eng, "prefill", refuse)
+    _check("small", eng, orc, 70, 5, seed=71, chunk=32 if chunk == "no memory" else chunk)
+    assert len(asked) == (chunk == "no memory")
 
 
 @pytest.mark.parametrize("name,n,pos", [("tiny", 1000, 0), ("tiny", 40, 900), ("tiny", 20, 1000), ("flint-3b-l1", 100, 2000),

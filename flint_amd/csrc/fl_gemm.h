@@ -1,9 +1,9 @@
 // int4 x bf16 GEMM for many activation rows (prompts): Y[M, N] = X[M, K] . dq[N, K]^T on the matrix
 // cores, the weights dequantised straight into MFMA operands, never written back as bf16.
 //
-// A workgroup of KW ways of NW waves computes BN = 16 NW NB weight rows x BM = 16 MB activation rows,
+// A workgroup of KW ways of NW waves computes BN = 16 NW weight rows x BM = 16 MB activation rows,
 // each way over its part of the K groups (the ways' sums meet in LDS, in way order). Wave w of a way
-// owns weight rows [16 NB w, 16 NB (w + 1)) of the tile, so no weight is dequantised twice in a
+// owns weight rows [16 w, 16 (w + 1)) of the tile, so no weight is dequantised twice in a
 // workgroup and the weights need no LDS; X is what a way's waves share: one 128-group of its BM rows
 // at a time in LDS, double-buffered, the next group's X and weights in flight in registers
 // meanwhile (one barrier per group). Weights are the MFMA's A operand, so a lane ends with four
@@ -74,11 +74,12 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& a, int& u, int& mb) {
 
 // Epi(n, m, v, split): v[i] = the (partial) sum of weight row n + i and activation row m; n is a
 // multiple of 4, rows past N or M are not filtered out.
-template <bool TILED, int NW, int KW, int NB, int MB, int WD, int XD, class Epi>
+template <bool TILED, int NW, int KW, int MB, int WD, int XD, class Epi>
 __global__ __launch_bounds__(64 * NW * KW, NW * KW > 8 ? 4 : 2) void k_gemm_rows(GemmArgs a, Epi epi) {
-  constexpr int BN = 16 * NW * NB, BM = 16 * MB;
+  static_assert((WD == 1 || WD == 2) && (XD == 1 || XD == 2), "groups requested ahead");
+  constexpr int BN = 16 * NW, BM = 16 * MB;
   constexpr int RP = 4 * NW, XI = BM / RP;  // X rows per pass of a way's threads, passes
-  constexpr int RED = (KW - 1) * NW * 64 * NB * MB * 16;  // the ways' sums, in X's place at the end
+  constexpr int RED = (KW - 1) * NW * 64 * MB * 16;  // the ways' sums, in X's place at the end
   constexpr int XS = KW * 2 * BM * 256;
   __shared__ __align__(16) unsigned char smem[XS > RED ? XS : RED];
   const int lane = threadIdx.x & 63, r = lane & 15, c = lane >> 4;
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(64 * NW * KW, NW * KW > 8 ? 4 : 2) void k_gemm_rows
   int u, mb;
   if (!gemm_tile(a, u, mb)) return;
   const int split = u % a.splits, G = a.k >> 7;
-  const int m0 = mb * BM, n0 = (u / a.splits) * BN + wave * (16 * NB);
+  const int m0 = mb * BM, n0 = (u / a.splits) * BN + wave * 16;
   // this way's groups; every way passes the same number of barriers
   const int gs0 = split * a.gps, gs1 = min(G, gs0 + a.gps), per = (gs1 - gs0 + KW - 1) / KW;
   const int g0 = gs0 + way * per, g1 = min(gs1, g0 + per);
@@ -101,17 +102,13 @@ __global__ __launch_bounds__(64 * NW * KW, NW * KW > 8 ? 4 : 2) void k_gemm_rows
   const uint32_t xstep = (uint32_t)a.k * (2u * RP);
   const uint32_t woff = TILED ? (uint32_t)(n0 >> 4) * (uint32_t)G * 1024u + (uint32_t)lane * 16u
                               : (uint32_t)(n0 + r) * (uint32_t)(a.k >> 1) + (uint32_t)c * 16u;
-  const uint32_t wstep = TILED ? (uint32_t)G * 1024u : (uint32_t)a.k * 8u;  // 16 rows, bytes
   const uint32_t soff = (uint32_t)(n0 + r) * (uint32_t)G * 4u;
   // requested ahead: the weights of WD groups, X of XD (past the way's last group: no memory access)
-  uint4 xv[XD][XI], wv[WD][NB];
-  uint32_t sv[WD][NB];
-  auto load_w = [&](int g, uint4 (&w)[NB], uint32_t (&s)[NB]) {
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      w[b] = buf_ld128(wr, g < g1 ? woff + (uint32_t)b * wstep + (uint32_t)g * (TILED ? 1024u : 64u) : 0xFFFFFFF0u);
-      s[b] = buf_ld32(sr, g < g1 ? soff + (uint32_t)b * (uint32_t)G * 64u + (uint32_t)g * 4u : 0xFFFFFFF0u);
-    }
+  uint4 xv[XD][XI], wv[WD];
+  uint32_t sv[WD];
+  auto load_w = [&](int g, uint4& w, uint32_t& s) {
+    w = buf_ld128(wr, g < g1 ? woff + (uint32_t)g * (TILED ? 1024u : 64u) : 0xFFFFFFF0u);
+    s = buf_ld32(sr, g < g1 ? soff + (uint32_t)g * 4u : 0xFFFFFFF0u);
   };
   auto load_x = [&](int g, uint4 (&x)[XI]) {
 #pragma unroll
@@ -136,11 +133,9 @@ __global__ __launch_bounds__(64 * NW * KW, NW * KW > 8 ? 4 : 2) void k_gemm_rows
       }
     }
   };
-  fl_f32x4 acc[NB][MB];
+  fl_f32x4 acc[MB];
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int i = 0; i < MB; ++i) acc[b][i] = fl_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int i = 0; i < MB; ++i) acc[i] = fl_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const MxLane mx = mx_lane();
   load_x(g0, xv[0]);
 #pragma unroll
@@ -151,125 +146,83 @@ __global__ __launch_bounds__(64 * NW * KW, NW * KW > 8 ? 4 : 2) void k_gemm_rows
   // one group: its operands are in wv[s] and LDS buffer s & 1
   auto group = [&](auto stage, int g) {
     constexpr int s = decltype(stage)::value, buf = s & 1;
-    uint4 wc[NB];
-    uint32_t sc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      wc[b] = wv[s % WD][b];
-      sc[b] = sv[s % WD][b];
-    }
+    const uint4 wc = wv[s % WD];
+    const uint32_t sc = sv[s % WD];
     lds_barrier();
     load_w(g + WD, wv[s % WD], sv[s % WD]);
     load_x(g + XD, xv[s % XD]);
     if (KW > 1 && g >= g1) return;  // fewer groups than the other ways: its barriers only
     const unsigned char* xrow = xs[buf] + r * 256;
-    auto mma = [&](int slot, const uint4 (&w)[NB]) {
+    auto mma = [&](int slot, const uint4 w) {
 #pragma unroll
       for (int i = 0; i < MB; ++i) {
         const uint4 xf = *reinterpret_cast<const uint4*>(xrow + i * 4096 + ((slot ^ r) * 16));
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-          acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(fl_bf16x8, w[b]),
-                                                              __builtin_bit_cast(fl_bf16x8, xf), acc[b][i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(fl_bf16x8, w),
+                                                         __builtin_bit_cast(fl_bf16x8, xf), acc[i], 0, 0, 0);
       }
     };
     if constexpr (TILED) {
-      // unit_dq_t's two exact steps, tiles 2tp, 2tp + 1 of every block together
-      fl_s16x4 bs[NB];
-      fl_f32x4 c1[NB], c2[NB];
+      // unit_dq_t's two exact steps, tiles 2tp, 2tp + 1 together
       const fl_s16x4 ai = mx_s4(0x3F803F80u & mx.mlo, 0x3F803F80u & mx.mhi);
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const uint32_t sb = sc[b] & 0xFFFFu, sp = sb | (sb << 16);
-        bs[b] = mx_s4(sp & mx.mlo, sp & mx.mhi);
-        const float c1v = -136.0f * bf2f(sb), zv = bf2f(sc[b] >> 16);
-        c1[b] = fl_f32x4{c1v, c1v, c1v, c1v};
-        c2[b] = fl_f32x4{zv, zv, zv, zv};
-      }
+      const uint32_t sb = sc & 0xFFFFu, sp = sb | (sb << 16);
+      const fl_s16x4 bs = mx_s4(sp & mx.mlo, sp & mx.mhi);
+      const float c1v = -136.0f * bf2f(sb), zv = bf2f(sc >> 16);
+      const fl_f32x4 c1 = {c1v, c1v, c1v, c1v}, c2 = {zv, zv, zv, zv};
+      const uint32_t v[4] = {wc.x, wc.y, wc.z, wc.w};
 #pragma unroll
       for (int tp = 0; tp < 4; ++tp) {
-        fl_f32x4 d[NB][2];
+        fl_f32x4 d[2];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          const uint32_t v[4] = {wc[b].x, wc[b].y, wc[b].z, wc[b].w};
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const int t = 2 * tp + e;
-            const uint32_t lo = v[t >> 2] >> (4 * (t & 3)), hi = v[2 + (t >> 2)] >> (4 * (t & 3));
-            d[b][e] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(
-                mx_s4((lo & mx.mask) | mx.magic, (hi & mx.mask) | mx.magic), bs[b], c1[b], 0, 0, 0);
-          }
+        for (int e = 0; e < 2; ++e) {
+          const int t = 2 * tp + e;
+          const uint32_t lo = v[t >> 2] >> (4 * (t & 3)), hi = v[2 + (t >> 2)] >> (4 * (t & 3));
+          d[e] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(mx_s4((lo & mx.mask) | mx.magic, (hi & mx.mask) | mx.magic),
+                                                        bs, c1, 0, 0, 0);
         }
-        uint32_t p[NB][2][2];
+        uint32_t p[2][2];
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
+        for (int e = 0; e < 2; ++e) {
+          p[e][0] = pack_bf16x2(d[e][0], d[e][1]);
+          p[e][1] = pack_bf16x2(d[e][2], d[e][3]);
+        }
 #pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            p[b][e][0] = pack_bf16x2(d[b][e][0], d[b][e][1]);
-            p[b][e][1] = pack_bf16x2(d[b][e][2], d[b][e][3]);
-          }
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-#pragma unroll
-          for (int e = 0; e < 2; ++e)
-            d[b][e] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ai, mx_s4(p[b][e][0], p[b][e][1]), c2[b], 0, 0, 0);
-        uint4 w[NB];
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-          w[b] = make_uint4(pack_bf16x2(d[b][0][0], d[b][0][1]), pack_bf16x2(d[b][0][2], d[b][0][3]),
-                            pack_bf16x2(d[b][1][0], d[b][1][1]), pack_bf16x2(d[b][1][2], d[b][1][3]));
-        mma(4 * tp + c, w);
+        for (int e = 0; e < 2; ++e) d[e] = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ai, mx_s4(p[e][0], p[e][1]), c2, 0, 0, 0);
+        mma(4 * tp + c, make_uint4(pack_bf16x2(d[0][0], d[0][1]), pack_bf16x2(d[0][2], d[0][3]),
+                                   pack_bf16x2(d[1][0], d[1][1]), pack_bf16x2(d[1][2], d[1][3])));
       }
     } else {
-      uint32_t d[NB][4][4];
+      uint32_t d[4][4];
+      dq32(wc, dq_const(sc), d);
 #pragma unroll
-      for (int b = 0; b < NB; ++b) dq32(wc[b], dq_const(sc[b]), d[b]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        uint4 w[NB];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) w[b] = make_uint4(d[b][0][e], d[b][1][e], d[b][2][e], d[b][3][e]);
-        mma(4 * c + e, w);
-      }
+      for (int e = 0; e < 4; ++e) mma(4 * c + e, make_uint4(d[0][e], d[1][e], d[2][e], d[3][e]));
     }
     if (g + 1 < g1) store(buf ^ 1, xv[(s + 1) % XD]);
   };
-  constexpr int UN = WD < 2 ? 2 : WD;  // the loop unrolled so that every buffer's index is fixed
-  for (int g = g0; g < g0 + per; g += UN) {
+  for (int g = g0; g < g0 + per; g += 2) {  // by two, so that every buffer's index is fixed
     group(std::integral_constant<int, 0>{}, g);
     if (g + 1 < g0 + per) group(std::integral_constant<int, 1>{}, g + 1);
-    if constexpr (UN > 2) {
-      if (g + 2 < g0 + per) group(std::integral_constant<int, 2>{}, g + 2);
-      if (g + 3 < g0 + per) group(std::integral_constant<int, 3>{}, g + 3);
-    }
   }
   if constexpr (KW > 1) {  // the ways' sums, added in way order
     lds_barrier();
     fl_f32x4* red = reinterpret_cast<fl_f32x4*>(smem);
     if (way > 0) {
 #pragma unroll
-      for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int i = 0; i < MB; ++i) red[((way - 1) * NB * MB + b * MB + i) * (NW * 64) + tid] = acc[b][i];
+      for (int i = 0; i < MB; ++i) red[((way - 1) * MB + i) * (NW * 64) + tid] = acc[i];
     }
     lds_barrier();
     if (way > 0) return;
 #pragma unroll
     for (int k = 0; k < KW - 1; ++k)
 #pragma unroll
-      for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int i = 0; i < MB; ++i) acc[b][i] += red[(k * NB * MB + b * MB + i) * (NW * 64) + tid];
+      for (int i = 0; i < MB; ++i) acc[i] += red[(k * MB + i) * (NW * 64) + tid];
   }
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
-#pragma unroll
-    for (int i = 0; i < MB; ++i) epi(n0 + 16 * b + 4 * c, m0 + 16 * i + r, acc[b][i], split);
+  for (int i = 0; i < MB; ++i) epi(n0 + 4 * c, m0 + 16 * i + r, acc[i], split);
 }
 
 typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
 
-// The same product for calls of many tiles: BN = 32 NW weight rows x BM = 32 TB activation rows per
+// The same product for calls of many tiles: BN = 32 NW weight rows x BM = 128 activation rows per
 // workgroup, on 32x32x16 MFMAs. A wave dequantises the operand of the next MFMA step (32 rows x 16 k)
 // between the MFMAs of the current one, and reads its X fragments a step ahead, in that order
 // (sched_barrier): beside 32x32 MFMAs the vector ALUs keep 0.9 of their rate (0.6 beside 16x16 ones), and a
@@ -280,8 +233,9 @@ typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
 // 1024 x 16384 x 2560: tiled 101 us, row 108 (k_gemm_rows with 128 x 128 tiles: 115, 128); 512: 53, 56 (57, 67).
 // What is left (timing builds of the tiled form, 118 us there): the MFMAs alone 63 us, which is 1.5
 // PFLOP/s, the rate that this card holds on any product; without the dequantisation 82; without storing X to LDS 99.
-template <bool TILED, int NW, int TB, class Epi>
+template <bool TILED, int NW, class Epi>
 __global__ __launch_bounds__(64 * NW, 2) void k_gemm_big(GemmArgs a, Epi epi) {
+  constexpr int TB = 4;  // 32-row tiles of X
   constexpr int BN = 32 * NW, BM = 32 * TB, RP = 4 * NW, XI = BM / RP;
   __shared__ __align__(16) unsigned char xs[2][BM * 256];
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, c = lane >> 4, r32 = lane & 31, h = lane >> 5;
@@ -426,10 +380,10 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_big(GemmArgs a, Epi epi) {
         __builtin_amdgcn_sched_barrier(0);
         acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fl_bf16x8, wq), __builtin_bit_cast(fl_bf16x8, xf[i]), acc[i], 0, 0, 0);
         xn[i] = s < 7 ? rd(buf, s + 1, i) : rd(buf ^ 1, 0, i);
-        if (i * 4 / TB == 0 && (i == 0 || TB < 4)) dq1(s < 7 ? (s + 1) >> 2 : 0, (s + 1) & 3);
-        if (i == TB / 4) { if (TB >= 4) dq2(); }
-        if (i == TB / 2) { if (TB < 4) dq2(); dq3(); }
-        if (i == TB - 1) wn = dq4();
+        if (i == 0) dq1(s < 7 ? (s + 1) >> 2 : 0, (s + 1) & 3);
+        if (i == 1) dq2();
+        if (i == 2) dq3();
+        if (i == 3) wn = dq4();
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

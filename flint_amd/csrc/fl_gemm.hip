@@ -80,16 +80,16 @@ Plan plan_rows(int m, int n, int k) {
   return p;
 }
 
-template <int NW, int KW, int NB, int MB, class Epi>
+template <int NW, int KW, int MB, class Epi>
 void launch(GemmArgs a, Epi epi, hipStream_t s) {
-  a.tile(16 * NW * NB, 16 * MB);
-  hipLaunchKernelGGL((k_gemm_rows<false, NW, KW, NB, MB, 1, 1, Epi>), dim3(gemm_grid(a)), dim3(64 * NW * KW), 0, s, a, epi);
+  a.tile(16 * NW, 16 * MB);
+  hipLaunchKernelGGL((k_gemm_rows<false, NW, KW, MB, 1, 1, Epi>), dim3(gemm_grid(a)), dim3(64 * NW * KW), 0, s, a, epi);
 }
 template <class Epi>
 void launch_small(int ways, const GemmArgs& a, Epi epi, hipStream_t s) {
-  if (ways == 4) launch<4, 4, 1, 4>(a, epi, s);
-  else if (ways == 2) launch<4, 2, 1, 4>(a, epi, s);
-  else launch<4, 1, 1, 4>(a, epi, s);
+  if (ways == 4) launch<4, 4, 4>(a, epi, s);
+  else if (ways == 2) launch<4, 2, 4>(a, epi, s);
+  else launch<4, 1, 4>(a, epi, s);
 }
 
 // The former kernel of 2 to 32 rows, kept for few K groups: one workgroup of four waves per 16 weight rows,
@@ -192,14 +192,14 @@ int fl_gemm_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint1
   if (few_groups(m, t16, k / FL_GROUP)) {
     hipLaunchKernelGGL(k_gemm, dim3(t16), dim3(64 * kGemmWaves), 0, s, q, sz, x, y, m, n, k);
   } else if (m <= 16) {
-    if (t16 <= 256) launch<1, 16, 1, 1>(a, epi, s);
-    else if (t16 <= 512) launch<2, 8, 1, 1>(a, epi, s);
-    else if (t16 <= 768) launch<1, 4, 1, 1>(a, epi, s);
-    else launch<2, 4, 1, 1>(a, epi, s);
+    if (t16 <= 256) launch<1, 16, 1>(a, epi, s);
+    else if (t16 <= 512) launch<2, 8, 1>(a, epi, s);
+    else if (t16 <= 768) launch<1, 4, 1>(a, epi, s);
+    else launch<2, 4, 1>(a, epi, s);
   } else {
-    if (t16 <= 256) launch<1, 8, 1, 2>(a, epi, s);
-    else if (t16 <= 512) launch<2, 8, 1, 2>(a, epi, s);
-    else launch<2, 4, 1, 2>(a, epi, s);
+    if (t16 <= 256) launch<1, 8, 2>(a, epi, s);
+    else if (t16 <= 512) launch<2, 8, 2>(a, epi, s);
+    else launch<2, 4, 2>(a, epi, s);
   }
   return hipGetLastError() == hipSuccess ? FL_OK : FL_E_LAUNCH;
 }
@@ -231,7 +231,7 @@ int fl_gemm_rows_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, 
     if (p.big) {
       GemmArgs b = a;
       b.tile(256, 128);
-      hipLaunchKernelGGL((k_gemm_big<false, 8, 4, EpiBf16>), dim3(gemm_grid(b)), dim3(512), 0, s, b, epi);
+      hipLaunchKernelGGL((k_gemm_big<false, 8, EpiBf16>), dim3(gemm_grid(b)), dim3(512), 0, s, b, epi);
     } else if (p.splits == 1) {
       launch_small(p.ways, a, epi, s);
     } else {

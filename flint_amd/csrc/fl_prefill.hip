@@ -454,10 +454,10 @@ template <int NW, int KW, int MB, class Epi>
 void pf_launch(GemmArgs a, Epi epi, hipStream_t s) {
   a.tile(16 * NW, 16 * MB);
   constexpr int D = KW == 1 ? 2 : 1;  // groups requested ahead
-  hipLaunchKernelGGL((k_gemm_rows<true, NW, KW, 1, MB, D, D, Epi>), dim3(gemm_grid(a)), dim3(64 * NW * KW), 0, s, a, epi);
+  hipLaunchKernelGGL((k_gemm_rows<true, NW, KW, MB, D, D, Epi>), dim3(gemm_grid(a)), dim3(64 * NW * KW), 0, s, a, epi);
 }
 
-// One GEMM of a pass. `parts`: the epilogue keeps fp32 sums of K parts, which k_pf_norm adds;
+// One GEMM of a pass. PARTS: the epilogue keeps fp32 sums of K parts, which k_pf_norm adds;
 // returns their number. Measured at flint-3b's sizes (us, weights from HBM):
 // - tiles of 256 x 128 (k_gemm_big, one workgroup per CU) where they and the parts give at least 160
 //   workgroups: gate/up at 512 / 1024 tokens (256 / 512 tiles) 53 / 101, 57 / 115 in tiles of 128 x 128; down at
@@ -469,29 +469,32 @@ void pf_launch(GemmArgs a, Epi epi, hipStream_t s) {
 //   groups, four at most, more while they give fewer than 160 workgroups: O at 512 (320 tiles) 19 in two parts,
 //   at 64 tokens 8 in four; down at 64 tokens 11 in four with four ways, 16 with one;
 // - tiles of 128 x 128 in between: QKV at 1024 (224 tiles) 39.
-template <class Epi>
-int pf_gemm(const uint32_t* qt, const uint32_t* sz, const uint16_t* x, int T, int n, int k, bool parts, Epi epi,
-            hipStream_t s) {
+template <bool PARTS, class Epi>
+int pf_gemm(const uint32_t* qt, const uint32_t* sz, const uint16_t* x, int T, int n, int k, Epi epi, hipStream_t s) {
   const int G = k / FL_GROUP;
   GemmArgs a{qt, sz, x, T, n, k, 0, 0, 1, G, 0};
-  const int t64 = ((n + 63) / 64) * ((T + 63) / 64), t128 = ((n + 127) / 128) * ((T + 127) / 128);
-  const int t256 = ((n + 255) / 256) * ((T + 127) / 128);
+  const int t64 = ((n + 63) / 64) * ((T + 63) / 64), t256 = ((n + 255) / 256) * ((T + 127) / 128);
   auto cut = [&](int want, int least) {  // K in `want` parts of at least `least` groups
     const int s = std::max(1, std::min({PF_SPLITS, want, G / least}));
     a.gps = (G + s - 1) / s;
     a.splits = (G + a.gps - 1) / a.gps;
   };
-  if (parts) cut(256 / t256, 8);
+  if (PARTS) cut(256 / t256, 8);
   const int big = t256 * a.splits;
   if (big >= 160 && (big <= 256 || big > 384)) {
     a.tile(256, 128);
-    hipLaunchKernelGGL((k_gemm_big<true, 8, 4, Epi>), dim3(gemm_grid(a)), dim3(512), 0, s, a, epi);
+    hipLaunchKernelGGL((k_gemm_big<true, 8, Epi>), dim3(gemm_grid(a)), dim3(512), 0, s, a, epi);
     return a.splits;
   }
-  if (parts) cut(std::max(G / 10, (160 + t64 - 1) / t64), 4);
+  if (PARTS) cut(std::max(G / 10, (160 + t64 - 1) / t64), 4);
+  if constexpr (!PARTS) {
+    if (((n + 127) / 128) * ((T + 127) / 128) >= 160) {
+      pf_launch<8, 1, 8>(a, epi, s);
+      return a.splits;
+    }
+  }
   const int wgs = t64 * a.splits;
-  if (!parts && t128 >= 160) pf_launch<8, 1, 8>(a, epi, s);
-  else if (wgs <= 256 && a.gps >= 8) pf_launch<4, 4, 4>(a, epi, s);
+  if (wgs <= 256 && a.gps >= 8) pf_launch<4, 4, 4>(a, epi, s);
   else if (wgs <= 512 && a.gps >= 8) pf_launch<4, 2, 4>(a, epi, s);
   else pf_launch<4, 1, 4>(a, epi, s);
   return a.splits;
@@ -539,18 +542,18 @@ void pf_pass(const fl_weights* w, fl_state* st, const PfWs& ws, const int32_t* t
                      w->attn_norm, d.norm_eps, ws.h, ws.xn, st->err);
   for (int l = 0; l < L; ++l) {
     const size_t layer = (size_t)l * d.n_kv_head * st->max_seq * 64;
-    pf_gemm(mat(w->wqkv_t, l, NQKV, D, 8), mat(w->wqkv_sz, l, NQKV, D, 128), ws.xn, T, NQKV, D, false,
-            EpiQkv{ws.q, st->kc + layer, st->vc + layer, reinterpret_cast<const uint32_t*>(w->rope), T, d.n_head,
-                   d.n_kv_head, st->max_seq, pos}, s);
+    pf_gemm<false>(mat(w->wqkv_t, l, NQKV, D, 8), mat(w->wqkv_sz, l, NQKV, D, 128), ws.xn, T, NQKV, D,
+                   EpiQkv{ws.q, st->kc + layer, st->vc + layer, reinterpret_cast<const uint32_t*>(w->rope), T, d.n_head,
+                          d.n_kv_head, st->max_seq, pos}, s);
     pf_attention(st, ws, l, T, pos, s);
-    int parts = pf_gemm(mat(w->wo_t, l, D, D, 8), mat(w->wo_sz, l, D, D, 128), ws.attn, T, D, D, true,
-                        EpiSum{ws.part, T, D}, s);
+    int parts = pf_gemm<true>(mat(w->wo_t, l, D, D, 8), mat(w->wo_sz, l, D, D, 128), ws.attn, T, D, D,
+                              EpiSum{ws.part, T, D}, s);
     hipLaunchKernelGGL(k_pf_norm, dim3(T), dim3(PF_NT), 0, s, ws.part, parts, T, D, tokens, w->embed, d.vocab,
                        d.resid_mult, w->ffn_norm + (size_t)l * D, d.norm_eps, ws.h, ws.xn, st->err);
-    pf_gemm(mat(w->wgu_t, l, 2 * F, D, 8), mat(w->wgu_sz, l, 2 * F, D, 128), ws.xn, T, 2 * F, D, false,
-            EpiSwiglu{ws.act, T, F}, s);
-    parts = pf_gemm(mat(w->wd_t, l, D, F, 8), mat(w->wd_sz, l, D, F, 128), ws.act, T, D, F, true,
-                    EpiSum{ws.part, T, D}, s);
+    pf_gemm<false>(mat(w->wgu_t, l, 2 * F, D, 8), mat(w->wgu_sz, l, 2 * F, D, 128), ws.xn, T, 2 * F, D,
+                   EpiSwiglu{ws.act, T, F}, s);
+    parts = pf_gemm<true>(mat(w->wd_t, l, D, F, 8), mat(w->wd_sz, l, D, F, 128), ws.act, T, D, F,
+                          EpiSum{ws.part, T, D}, s);
     const uint16_t* next = l + 1 < L ? w->attn_norm + (size_t)(l + 1) * D : w->final_norm;
     hipLaunchKernelGGL(k_pf_norm, dim3(T), dim3(PF_NT), 0, s, ws.part, parts, T, D, tokens, w->embed, d.vocab,
                        d.resid_mult, next, d.norm_eps, ws.h, ws.xn, st->err);

@@ -15,13 +15,15 @@
 // and barriers alone took 158 us, the dequantisation alone about 100. A v_dot2_f32_bf16 of the dequantisation
 // runs on the matrix pipe itself (measured: beside a wave that issues MFMAs it gets next to no slots, where a
 // v_fma_f32 keeps its rate), and other vector instructions issue at 0.6 of their rate beside 16x16 MFMAs.
-// Calls of many tiles take k_gemm_big below instead (195 us).
+// Calls of many tiles take k_gemm_big below instead (210 us).
 //
 // The ways are for calls of few tiles, where a group's memory latency, not its work, is what a step
 // costs: 32 rows x 16384 x 2560 (256 tiles) takes 20 steps of one way or 5 of four, 64 rows 19 and
 // 13 us; 512 x 3584 x 2560 (448 tiles) 28 us with one way and 21 with two.
 // Two groups requested ahead instead of one (WD, XD) gain 7-10% with one way on the tiled layout (2048 x
-// 16384 x 2560 222 -> 206 us), and lose with more ways (the registers cost a workgroup per CU).
+// 16384 x 2560 222 -> 206 us). They cost with more ways, though a CU holds as many workgroups then (LDS sets their
+// number): prompts of 64 / 512 tokens, 12 layers, 835 / 1901 us with one group ahead, 931 / 1924 with two; row layout 333 x
+// 2570 x 2560 17.5 and 21.3 (two of the weights alone 18.5), 5 x 2560 x 8192 13.6 and 14.8.
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -93,7 +95,8 @@ __global__ __launch_bounds__(64 * NW * KW, NW * KW > 8 ? 4 : 2) void k_gemm_rows
   // this way's groups; every way passes the same number of barriers
   const int gs0 = split * a.gps, gs1 = min(G, gs0 + a.gps), per = (gs1 - gs0 + KW - 1) / KW;
   const int g0 = gs0 + way * per, g1 = min(gs1, g0 + per);
-  // range-checked: rows past M or N read as zeros
+  // range-checked: rows past M or N read as zeros (or, in a matrix that almost fills 4 GB, where their 32-bit
+  // offset wraps, as its first rows: the epilogue drops them either way)
   const auto xr = buf_rsrc(a.x, (uint32_t)a.m * (uint32_t)a.k * 2u);
   const auto wr = buf_rsrc(a.q, (uint32_t)a.n * (uint32_t)(a.k >> 1));
   const auto sr = buf_rsrc(a.sz, (uint32_t)a.n * (uint32_t)G * 4u);
@@ -231,7 +234,8 @@ typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
 // tiled layout holds that; from the row layout a lane loads the word it needs of each of its four rows
 // (4-byte loads) and pairs their halves, and takes columns 8 apart in a step, which X in LDS follows.
 // 1024 x 16384 x 2560: tiled 101 us, row 108 (k_gemm_rows with 128 x 128 tiles: 115, 128); 512: 53, 56 (57, 67).
-// What is left (timing builds of the tiled form, 118 us there): the MFMAs alone 63 us, which is 1.5
+// 2048: row 210, 0.82 PFLOP/s, the matrix pipes busy for 0.48 of the cycles.
+// What is left (timing builds of the tiled form at 1024, 118 us there): the MFMAs alone 63 us, which is 1.5
 // PFLOP/s, the rate that this card holds on any product; without the dequantisation 82; without storing X to LDS 99.
 template <bool TILED, int NW, class Epi>
 __global__ __launch_bounds__(64 * NW, 2) void k_gemm_big(GemmArgs a, Epi epi) {

@@ -42,23 +42,20 @@ __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ p, 
   out(nn, mm, v, 0);
 }
 
-// How a call of m rows runs. Tiles of 128 rows x 256 weight rows (k_gemm_big, one workgroup per CU) where
-// they nearly fill the 256 CUs: 512 / 2048 rows x 16384 x 2560 56 / 201 us, 64 x 64 tiles 89 / 340. A second round that
-// is half empty still costs a whole one, which up to 12 groups is more than the smaller tiles take: 576 rows x
-// 16384 (320 tiles) x 640 35 and 31, x 1280 54 and 52, x 2560 92 and 97; 700 x 12288 (288) x 1280 54 and 49; 768 x 16384
-// (384) x 640 37 and 38; one or two groups do not pay for the large tiles' start-up: 448 x 12288 x 256 15 and 14.
-// Else 64 x 64 tiles; a CU holds one workgroup of four ways, two of two, three of one (us, weights from HBM):
-// - up to 256 tiles four ways (two where a part has fewer than 8 groups), and K cut while all parts' tiles still run at
-//   once: 333 x 2570 x 2560 (246 tiles) 25 with one way, 17 with two, 16 with four, 20 with one way in 2
-//   parts, whose sums cost a launch; 100 x 3584 x 2560 (112) 15 uncut, 13 in 2 parts; 64 x 2560 x 8192
-//   (40) 36 uncut with one way, 12 in 4 parts;
-// - beyond 32 groups, where those leave CUs idle (129 to 200 tiles) or there are more tiles: parts of one
-//   way for about 1536 workgroups: 200 x 2560 x 8192 (160 tiles) 34 in 4 parts, 38 with four ways; 333 x 2900
-//   x 8192 (276) 52 in 4 parts, 57 in 2, 66 with two ways; 600 x 3584 x 8192 (560) 93 in 2, 100 uncut; of
-//   12 groups at least: 97 x 12260 x 4224 (384, 33 groups) 43 in 4 parts, 40 in 2;
-// - else two ways, one beyond 512 tiles of at most 16 groups: 333 x 2900 x 2560 (276) 26 with one way, 23 with
-//   two, 24 in parts; 100 x 16384 x 2560 (512) 31 and 26, 2048 x 2560 x 2560 (1280) 58 and 56;
-//   389 x 11621 x 640 (1274) 22 and 24, 1355 x 10528 x 1024 (3630) 49 and 66.
+// How a call of m rows runs (us, weights from HBM).
+// Large tiles, 128 rows x 256 weight rows (k_gemm_big, one workgroup per CU): from 224 of them on, but not where a
+// second round would be half empty or more (257 to 383) at up to 12 groups, which the smaller tiles outrun, nor for one
+// or two groups, which do not pay for its start-up. 512 x 16384 x 2560 (256) 56, in 64 x 64 tiles 89; 576 x 16384
+// (320) x 640 35 and 31, x 1280 54 and 52, x 2560 92 and 97; 768 x 16384 (384) x 640 37 and 38; 448 x 12288 x 256 15 and 14.
+// Else 64 x 64 tiles; a CU holds one workgroup of four ways, two of two (LDS), five of one (registers):
+// - few tiles (up to 256; beyond 32 groups not 129 to 200, which leave CUs idle): four ways, two where a part has fewer
+//   than 8 groups, and K cut while all parts' tiles still run at once. 333 x 2570 x 2560 (246 tiles) 16, with two ways
+//   17, one 25, one in 2 parts, whose sums cost a launch, 20; 100 x 3584 x 2560 (112) 13 in 2 parts, 15 uncut;
+// - more, beyond 32 groups: one way, parts of at least 12 groups for about 1536 workgroups. 200 x 2560 x 8192 (160) 34 in
+//   4 parts, 38 with four ways; 333 x 2900 x 8192 (276) 52, in 2 parts 57, with two ways 66; 600 x 3584 x 8192
+//   (560) 93 in 2, 100 uncut; 97 x 12260 x 4224 (384, 33 groups) 40 in 2, 43 in 4;
+// - more, up to 32 groups: two ways, one beyond 512 tiles of at most 16 groups. 333 x 2900 x 2560 (276) 23, with one
+//   26; 2048 x 2560 x 2560 (1280) 56 and 58; 389 x 11621 x 640 (1274) 24 and 22.
 struct Plan {
   bool big;
   int ways, splits, gps;
@@ -162,7 +159,8 @@ EpiBf16 out_bf16(uint16_t* y, int m, int n) {
   return EpiBf16{y, m, n, n % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0};
 }
 
-// rows of one launch: 32-bit byte offsets over X (and the rows of a last tile past its end)
+// rows of one launch: 32-bit byte offsets over X and the rows of a last tile past its end; over the weights up to the
+// matrix's own end (the rows of a 256-row tile past it may wrap, within the matrix, and are dropped)
 constexpr int ROWS_PER_LAUNCH = 8192;
 bool rows_ok(int n, int k) {
   return k <= 65536 && ((int64_t)n + 128) * (k / 2) <= 0xFFFFFFFFll;

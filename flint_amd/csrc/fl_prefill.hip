@@ -6,8 +6,8 @@
 //   residual + RMSNorm -> gate/up GEMM (SwiGLU in its epilogue) -> down GEMM -> residual + RMSNorm,
 // the O and down GEMMs cut along K into fp32 part sums that the residual kernel adds in order. After
 // the last pass the LM head and argmax of the last token.
-// At 512 tokens of flint-3b a layer takes 151 us (of which the GEMMs: QKV 24, O 19, gate/up 52, down 38;
-// attention 12, the two norms 13), against 1336 in sixteen k_verify launches; 40 tokens take 64 us a
+// At 512 tokens of flint-3b a layer takes 152 us (of which the GEMMs: QKV 22, O 18, gate/up 51, down 36;
+// attention 11, the two norms 14), against 1336 in sixteen k_verify launches; 40 tokens take 64 us a
 // layer (launches and latency) against 120, and up to 16 they take the one k_verify launch (16: 46 us a
 // layer against 62; 24: 71 against 62, at 12000 cached keys 118 against 85).
 #include "fl_gemm.h"

@@ -12,8 +12,8 @@ constexpr uint32_t kBf16OneEMinus6 = 0x3586u;  // bf16(1e-6): clamp(min=1e-6) on
 
 // Eight threads per (row, 128-group), two packed words (8 elements each) per thread. Bound by
 // the vector ALUs as much as by HBM: with a full division per element and LDS shuffles 16384 x
-// 2560 took 36.6 us (2.9 TB/s); one word per thread without either 29.9, two (half the group arithmetic) 21.7
-// us (4.9 TB/s).
+// 2560 took 36.6 us (2.9 TB/s); one word per thread without either 29.9, two (half the group arithmetic) 21
+// us (5.1 TB/s).
 // t / scale, correctly rounded, without a division: y = RN(1 / scale) once, then q0 = RN(t y), r = t -
 // q0 scale (exact) and q1 = RN(q0 + r y). q0 is within 1.5 ulp of the quotient, so q0 + r y is within
 // 2^-23 ulp of it, and the quotient of two bf16 values lies at least 2^-9 ulp from every midpoint of

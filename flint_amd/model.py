@@ -284,7 +284,7 @@ class Transformer:
     def prefill(self, tokens, pos, token_out):
         """A prompt (int32 device [n]) at cache slots pos..pos+n-1 in passes of up to 1024 tokens
         (fl_prefill): fills the cache and writes the greedy next token to token_out (int32 device
-        [1]), which it returns. The workspace (84 MB for 1024 tokens of flint-3b) is torch's."""
+        [1]), which it returns. The workspace (80 MB for 1024 tokens of flint-3b) is torch's."""
         if self._state is None:
             raise RuntimeError("call setup_caches first")
         tokens = tokens.contiguous()

@@ -103,8 +103,8 @@ int fl_gemv_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint1
 int fl_gemm_int4(const uint32_t* q, const uint32_t* sz, const uint16_t* x, uint16_t* y,
                  int32_t m, int32_t n, int32_t k, void* stream);
 
-/* The same product for any M >= 1 (a whole prompt through one layer): tiles of 64 or 128 rows of
- * both operands on the matrix cores, each weight dequantised once per 64 or 128 rows of X. ws: device
+/* The same product for any M >= 1 (a whole prompt through one layer): tiles of 64 rows of both operands,
+ * or of 256 weight rows and 128 rows of X, on the matrix cores, each weight dequantised once per tile. ws: device
  * workspace of at least the bytes that fl_gemm_rows_workspace gives for (m, n, k) (0: may be NULL),
  * 16-byte aligned, free for reuse once the call's work on the stream is done. FL_E_ARG for a size
  * that they do not take (K > 65536, or N K / 2 beyond 4 GB).
@@ -221,7 +221,7 @@ int fl_verify(const fl_weights* w, fl_state* st, const int32_t* tokens, int32_t 
  * into the cache, the greedy next token after the last one to *token_out. The same operations as
  * fl_verify, in ordinary launches over up to 1024 tokens at a time; it takes the models that
  * fl_verify takes and needs the tiled weight copies. workspace: device memory of the bytes that
- * fl_prefill_workspace gives for n (84 MB for 1024 tokens of flint-3b), 256-byte aligned, free for
+ * fl_prefill_workspace gives for n (80 MB for 1024 tokens of flint-3b), 256-byte aligned, free for
  * reuse once the call's work on the stream is done. tokens / token_out are device pointers; a
  * token id outside the vocabulary is recorded in the state (fl_state_check). Nothing is allocated, and
  * a captured call replays (no tags).

@@ -9,7 +9,7 @@ runs as GEMM passes over up to 1024 tokens (fl_prefill), a short one through the
 import torch
 
 # prompts of more tokens than this run as fl_prefill passes: up to 16 tokens are one token pass of the verify
-# launch (flint-3b, 40 layers: 16 tokens 1.8 ms against 2.5 in a pass, 24 tokens 2.8 against 2.5)
+# launch (flint-3b, 40 layers: 16 tokens 1.8 ms against 2.6 in a pass, 24 tokens 2.8 against 2.6)
 PREFILL_MIN = 16
 
 
